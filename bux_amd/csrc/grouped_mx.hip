@@ -381,29 +381,50 @@ __device__ __forceinline__ void stream8(void* at, uint32_t x, uint32_t y) {
   __builtin_nontemporal_store(u32x2{x, y}, reinterpret_cast<u32x2*>(at));
 }
 
-// float32 (for tests), by every wave, straight from the accumulators: lane l holds row
-// l % 32 of each 32-row block and, in register run g, columns 8 g + 4 (l / 32) .. + 3 of
-// each 32-column block. The tile's rows [0, rows) and columns [0, cols) are stored (cols
-// a multiple of 4), at row pitch ld, from its corner.
-__device__ void store_f32(const v16f acc[4][4], float* tile, int32_t ld, int32_t rows, int32_t cols) {
+// float32 through the wave's region of the stage, 32 rows x 64 columns (a row's 256 bytes,
+// rows 272 apart) at a time: read back 16 bytes a lane, 16 lanes a row, a store writes
+// 4 whole rows of 256 bytes. (Straight from the accumulators a store instruction wrote
+// 32 rows of 32 bytes: config 3's up wgrad into float32, 1.6 GB of outputs, took 1494 us,
+// this way 627.) I, J: the wave's blocks of 32 rows and columns, its first row and column
+// row0 and col0 of the tile; the rows [0, rows) and columns [0, cols) are stored (cols a
+// multiple of 4).
+template <int I, int J>
+__device__ void store_f32(const v16f acc[4][4], float* tile, int32_t ld, int32_t rows, int32_t cols,
+                          int32_t row0, int32_t col0, Stage& stage) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
+  constexpr int FP = 272;
+  uint8_t* region = reinterpret_cast<uint8_t*>(&stage) + wave * 32 * FP;
+  uint8_t* mine = region + (lane & 31) * FP + 16 * (lane >> 5);
+  const int cc = lane & 15;
+  const uint8_t* from = region + (lane >> 4) * FP + cc * 16;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int32_t row = wm * 128 + i * 32 + (lane & 31);
-    if (row >= rows) continue;
+  for (int i = 0; i < I; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int jj = 0; jj < J; jj += 2) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int32_t col = wn * 128 + j * 32 + 8 * g + 4 * (lane >> 5);
-        const v16f& a = acc[i][j];
-        if (col < cols)
-          stream16(tile + row * ld + col,
-                   make_uint4(__float_as_uint(a[4 * g]), __float_as_uint(a[4 * g + 1]),
-                              __float_as_uint(a[4 * g + 2]), __float_as_uint(a[4 * g + 3])));
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const v16f& a = acc[i][jj + b];
+          *reinterpret_cast<float4*>(mine + b * 128 + g * 32) =
+              make_float4(a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]);
+        }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_wave_barrier();
+      uint4 v[8];
+#pragma unroll
+      for (int it = 0; it < 8; ++it) v[it] = *reinterpret_cast<const uint4*>(from + it * 4 * FP);
+      const int32_t col = col0 + jj * 32 + 4 * cc;
+      if (col < cols) {
+#pragma unroll
+        for (int it = 0; it < 8; ++it) {
+          const int32_t row = row0 + i * 32 + it * 4 + (lane >> 4);
+          if (row < rows) stream16(tile + row * ld + col, v[it]);
+        }
       }
-  }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_wave_barrier();
+    }
 }
 
 // bfloat16 through one stage of LDS, in 4 rounds of 32 rows: each wave puts its block of
@@ -490,8 +511,9 @@ __device__ __forceinline__ void store_tile(const v16f acc[4][4], uint16_t* tile,
   store_bf16(FromAcc{acc}, tile, ld, rows, cols, stage);
 }
 __device__ __forceinline__ void store_tile(const v16f acc[4][4], float* tile, int32_t ld,
-                                           int32_t rows, int32_t cols, Stage&) {
-  store_f32(acc, tile, ld, rows, cols);
+                                           int32_t rows, int32_t cols, Stage& stage) {
+  const int wave = threadIdx.x >> 6;
+  store_f32<4, 4>(acc, tile, ld, rows, cols, (wave >> 1) * 128, (wave & 1) * 128, stage);
 }
 
 // A half tile's outputs, each wave's 128 rows x 64 columns (columns 64 w on; accumulator
@@ -542,26 +564,11 @@ __device__ void store_tile_half(const v16f acc[4][4], uint16_t* tile, int32_t ld
     __builtin_amdgcn_wave_barrier();
   }
 }
-// float32 (for tests), straight from the accumulators as store_f32.
+// float32 as store_f32.
 __device__ void store_tile_half(const v16f acc[4][4], float* tile, int32_t ld, int32_t rows,
-                                int32_t cols, Stage&) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int32_t row = i * 32 + (lane & 31);
-    if (row >= rows) continue;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int32_t col = wave * 64 + j * 32 + 8 * g + 4 * (lane >> 5);
-        const v16f& a = acc[i][j];
-        if (col < cols)
-          stream16(tile + row * ld + col,
-                   make_uint4(__float_as_uint(a[4 * g]), __float_as_uint(a[4 * g + 1]),
-                              __float_as_uint(a[4 * g + 2]), __float_as_uint(a[4 * g + 3])));
-      }
-  }
+                                int32_t cols, Stage& stage) {
+  const int wave = threadIdx.x >> 6;
+  store_f32<4, 2>(acc, tile, ld, rows, cols, 0, wave * 64, stage);
 }
 
 // bfloat16 of a tile that stores every row and column (PH: a half tile's 128 rows),
