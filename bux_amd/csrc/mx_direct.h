@@ -1,0 +1,19 @@
+// The MXFP8 rows GEMM for short groups (mx_direct.hip): which calls it takes, and its
+// launch. grouped_mx.hip's launch asks first.
+#pragma once
+
+#include "common.h"
+
+namespace bux {
+
+// Whether a rows GEMM over `m` rows in `groups` groups goes to rows_direct_kernel.
+bool rows_direct(int64_t m, int32_t groups);
+
+// As grouped_mx.hip's launch_rows: `list` a tile list of `slots` records (its starts
+// before them), the operands in the tiled layout, y (height, n) of out_dtype.
+int launch_rows_direct(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b_values,
+                       const uint8_t* b_scales, const void* list, int64_t slots, int32_t groups,
+                       int64_t m, int64_t n, int64_t k, int64_t height, int out_dtype, void* y,
+                       hipStream_t s);
+
+}  // namespace bux

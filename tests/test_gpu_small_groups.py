@@ -1,6 +1,8 @@
-"""The MXFP8 GEMMs' float32 epilogue at the edges of its tiles: both dtypes store the same
-float32 sums, so a bfloat16 output is its float32 twin's rounding to the bit. (The values
-against the oracle's float64 sums: tests/test_gpu_gemm.py.)"""
+"""The MXFP8 GEMMs' float32 epilogue and the rows GEMM for groups of few rows, at the
+edges of their tiles, against each other: every output of either kernel is the same
+float32 sum, so a bfloat16 output is its float32 twin's rounding to the bit, and a call
+that goes to one rows kernel gives the other's bits. (Their values against the oracle's
+float64 sums: tests/test_gpu_gemm.py, whose cases take both kernels.)"""
 
 import numpy as np
 import pytest
@@ -18,6 +20,41 @@ def _codes(rng, shape):
         np.array([0, 128], np.uint8), (*lead, k // 64, r, 64))
     scales = rng.integers(118, 132, (*lead, k // 128, r, 4), np.uint8)
     return grouped_mxfp8.Tiled(torch.from_numpy(values).cuda(), torch.from_numpy(scales).cuda())
+
+
+# sizes, k, n: groups at and over a block of 32 rows, one of a whole tile and more, empty
+# ones, rows past the groups; n off the waves' 32 and 64 columns; K of one pair, of an odd
+# number of them, of fewer than are in flight
+SMALL = [
+    ([1] + [0] * 31, 128, 4),
+    ([5, 0, 32, 33, 1] + [0] * 45, 256, 132),
+    ([0, 300] + [1] * 60, 384, 260),
+    ([64, 31, 0, 7] + [2] * 60, 1152, 96),
+    ([3] * 128, 640, 1540),  # waves of 64 columns
+    ([0] * 20 + [40], 896, 160),
+]
+
+
+@pytest.mark.parametrize("sizes,k,n", SMALL)
+def test_rows_of_few_rows_are_the_tiled_kernels(lib, sizes, k, n):
+    from bux_amd import grouped_mxfp8
+    rng = np.random.default_rng(70)
+    groups, filled = len(sizes), sum(sizes)
+    m = filled + 3
+    assert m <= 20 * groups
+    far = 20 * groups + 1  # rows enough for the tiled kernel
+    a = _codes(rng, (far, k))
+    few = grouped_mxfp8.Tiled(a.values[:, :m].contiguous(), a.scales[:, :m].contiguous())
+    b = _codes(rng, (groups, n, k))
+    gs = torch.tensor(sizes, dtype=torch.int32, device="cuda")
+    announce("rows of few rows", sizes[:5], k, n)
+    got = [grouped_mxfp8.rows(few, b, gs, dt) for dt in (torch.bfloat16, torch.float32)]
+    want = [grouped_mxfp8.rows(a, b, gs, dt) for dt in (torch.bfloat16, torch.float32)]
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        assert torch.equal(g, w[:m])
+        assert (g[filled:] == 0).all()
+    assert torch.equal(got[0], got[1].to(torch.bfloat16))
 
 
 # group sizes, n (or d and f): whole tiles, half tiles, partial ones, columns of a multiple
