@@ -1434,7 +1434,7 @@ int launch_rows_of(const uint8_t* a_values, const uint8_t* a_scales, const uint8
   const int64_t slots = row_slots(groups, m, height);
   int32_t* starts = starts_in(list);
   Tile* tiles = tiles_in(list, groups);
-  if (rows_direct(m, groups))
+  if (rows_direct(m, groups, n))
     return launch_rows_direct(a_values, a_scales, b_values, b_scales, list, slots, groups, m, n, k,
                               height, out_dtype, y, s);
   return out_dtype == BUX_BF16

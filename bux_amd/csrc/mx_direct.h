@@ -6,8 +6,9 @@
 
 namespace bux {
 
-// Whether a rows GEMM over `m` rows in `groups` groups goes to rows_direct_kernel.
-bool rows_direct(int64_t m, int32_t groups);
+// Whether a rows GEMM of `m` rows in `groups` groups, `n` columns, goes to
+// rows_direct_kernel.
+bool rows_direct(int64_t m, int32_t groups, int64_t n);
 
 // As grouped_mx.hip's launch_rows: `list` a tile list of `slots` records (its starts
 // before them), the operands in the tiled layout, y (height, n) of out_dtype.

@@ -3,13 +3,15 @@
 // That file's schedule (one workgroup a CU on a 256 x 256 tile, operands shared through
 // LDS) has too few tiles there to fill the chip, and a tile of 5 rows costs it 128.
 //
-// Here a wave takes 32 rows by 32 CB columns of its own, its operands straight from global
-// memory to registers, two K pairs (256 bytes of K) ahead: no LDS, no barrier, no other
-// wave to wait for, and two to four waves a SIMD, so that one's epilogue runs beside
-// another's loads. The tiled layout serves that as it serves LDS: a block's 64-byte K
-// chunks are one run of 2 KiB. Loads four pairs ahead were no faster, non-temporal loads
-// of B 15-20% slower. Memory bounds it: 128 groups of K 2048, N 1536 at 4.6 (53 of them
-// with a row) to 5.5 TB/s (all of them).
+// Here a wave is a workgroup of its own and takes 32 rows by 64 columns, its operands
+// straight from global memory to registers, two K pairs (256 bytes of K) ahead: no LDS, no
+// barrier, no other wave to wait for, and two waves a SIMD, so that one's epilogue runs
+// beside another's loads. The tiled layout serves that as it serves LDS: a block's 64-byte
+// K chunks are one run of 2 KiB. What bounds it is each CU's loads in flight, so the waves
+// have to spread evenly over the CUs: in workgroups of four the unevenly loaded ones last
+// (16 groups of K 6400, N 4096, 32 rows on Zipf loads 60 -> 55 us, 96 rows 110 -> 85). Half
+// the columns a wave, four pairs ahead and non-temporal loads of B were all slower. 128
+// groups of K 2048, N 1536: 5.5 TB/s.
 //
 // The sums are grouped_mx.hip's to the bit (v_mfma_scale_f32_32x32x64_f8f6f4 over the K
 // steps in order, from 0), so that a call may go either way.
@@ -24,7 +26,9 @@ namespace {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 
-constexpr int WAVES = THREADS / 64;
+constexpr int BLOCK = 32;  // rows a wave
+constexpr int CB = 2;      // its blocks of 32 columns
+constexpr int D = 2;       // K pairs in flight
 
 // A 32-row block's operand registers of one MFMA (the lane's 16 bytes of each of the
 // step's two 32-byte blocks).
@@ -41,142 +45,136 @@ __device__ __forceinline__ uint4 load16(const uint8_t* base, uint32_t at) {
 
 // One K pair (128 bytes: two MFMA steps and one scale word a row) of a wave's block of A
 // and its CB blocks of B.
-template <int CB>
 struct Pair {
   uint4 a[4], b[CB][4];
   uint32_t sa, sb[CB];
 };
 
-// A workgroup takes one tile of the list (up to 256 rows) and 4 blocks of 32 CB columns:
-// the tile's blocks of 32 rows by those are its waves' jobs, row blocks fastest, so that
-// waves running together on a longer group share B's bytes through the L1.
-template <typename T, int CB>
-__global__ __launch_bounds__(THREADS) void rows_direct_kernel(
+// blockIdx.y: a tile's block of 32 rows; those past most tiles' rows leave at once, and come
+// last in the grid.
+template <typename T>
+__global__ __launch_bounds__(64) void rows_direct_kernel(
     const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_scales,
     const uint8_t* __restrict__ b_values, const uint8_t* __restrict__ b_scales, int32_t k,
     int32_t a_rows, int32_t n, int32_t groups, int32_t height, const int32_t* __restrict__ starts,
     const Tile* __restrict__ tiles, int32_t col_blocks, T* __restrict__ y) {
-  constexpr int D = 2;  // pairs in flight
   if (!list_fits(starts, groups, a_rows, height)) return;
   const int32_t id = blockIdx.x / col_blocks;
   if (id >= starts[groups + 1]) return;
   const Tile t = tiles[id];
-  const int32_t rows = smaller(t.hi, height) - t.lo;
-  if (rows <= 0) return;
-  const int lane = threadIdx.x & 63, half = lane >> 5, r32 = lane & 31;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int32_t row_blocks = (rows + 31) / 32;
+  const int32_t row0 = t.lo + static_cast<int32_t>(blockIdx.y) * BLOCK, end = smaller(t.hi, height);
+  if (row0 >= end) return;
+  const int lane = threadIdx.x, half = lane >> 5, r32 = lane & 31;
+  const int32_t col0 = (blockIdx.x % col_blocks) * 32 * CB;
   const int32_t pairs = t.group < groups ? k / 128 : 0;  // rows past the groups: zeros
   const int32_t group = t.group < groups ? t.group : 0;
   const uint8_t* const bv = b_values + static_cast<int64_t>(group) * n * k;
   const uint8_t* const bs = b_scales + static_cast<int64_t>(group) * n * (k / 32);
   const int64_t a_chunk = static_cast<int64_t>(a_rows) * 64, b_chunk = static_cast<int64_t>(n) * 64;
-  for (int32_t job = wave; job < row_blocks * WAVES; job += WAVES) {
-    const int32_t row0 = t.lo + (job % row_blocks) * 32;
-    const int32_t col0 = ((blockIdx.x % col_blocks) * WAVES + job / row_blocks) * 32 * CB;
-    if (col0 >= n) break;  // the next jobs' columns lie further
-    // rows past an operand's are its last one's again, and not stored
-    const uint32_t ar = static_cast<uint32_t>(smaller(row0 + r32, a_rows - 1));
-    uint32_t br[CB];
+  // rows past an operand's are its last one's again, and not stored
+  const uint32_t ar = static_cast<uint32_t>(smaller(row0 + r32, a_rows - 1));
+  uint32_t br[CB];
 #pragma unroll
-    for (int j = 0; j < CB; ++j) br[j] = static_cast<uint32_t>(smaller(col0 + 32 * j + r32, n - 1));
-    v16f acc[CB];
+  for (int j = 0; j < CB; ++j) br[j] = static_cast<uint32_t>(smaller(col0 + 32 * j + r32, n - 1));
+  v16f acc[CB];
+#pragma unroll
+  for (int j = 0; j < CB; ++j)
+#pragma unroll
+    for (int q = 0; q < 16; ++q) acc[j][q] = 0.0f;
+
+  Pair in[D];
+  auto load = [&](Pair& s, int32_t p) {
+    const uint8_t* a0 = a_values + 2 * p * a_chunk;
+    const uint8_t* b0 = bv + 2 * p * b_chunk;
+    const uint8_t* as0 = a_scales + static_cast<int64_t>(p) * a_rows * 4;
+    const uint8_t* bs0 = bs + static_cast<int64_t>(p) * n * 4;
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+      const uint32_t at = br[j] * 64 + 16 * half;
+      s.b[j][0] = load16(b0, at);
+      s.b[j][1] = load16(b0, at + 32);
+      s.b[j][2] = load16(b0 + b_chunk, at);
+      s.b[j][3] = load16(b0 + b_chunk, at + 32);
+      s.sb[j] = *reinterpret_cast<const uint32_t*>(bs0 + br[j] * 4);
+    }
+    const uint32_t at = ar * 64 + 16 * half;
+    s.a[0] = load16(a0, at);
+    s.a[1] = load16(a0, at + 32);
+    s.a[2] = load16(a0 + a_chunk, at);
+    s.a[3] = load16(a0 + a_chunk, at + 32);
+    s.sa = *reinterpret_cast<const uint32_t*>(as0 + ar * 4);
+  };
+  // Lane half h's scale byte is byte h of a word in its first step and 2 + h in its
+  // second: the word shifted by h bytes, the MFMA taking its byte 0, then 2.
+  auto multiply = [&](const Pair& s) {
+    const int wa = static_cast<int>(s.sa >> (8 * half));
+    int wb[CB];
+#pragma unroll
+    for (int j = 0; j < CB; ++j) wb[j] = static_cast<int>(s.sb[j] >> (8 * half));
 #pragma unroll
     for (int j = 0; j < CB; ++j)
+      acc[j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+          operand(s.b[j][0], s.b[j][1]), operand(s.a[0], s.a[1]), acc[j], 0, 0, 0, wb[j], 0, wa);
 #pragma unroll
-      for (int q = 0; q < 16; ++q) acc[j][q] = 0.0f;
-
-    Pair<CB> in[D];
-    auto load = [&](Pair<CB>& s, int32_t p) {
-      const uint8_t* a0 = a_values + 2 * p * a_chunk;
-      const uint8_t* b0 = bv + 2 * p * b_chunk;
-      const uint8_t* as0 = a_scales + static_cast<int64_t>(p) * a_rows * 4;
-      const uint8_t* bs0 = bs + static_cast<int64_t>(p) * n * 4;
+    for (int j = 0; j < CB; ++j)
+      acc[j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+          operand(s.b[j][2], s.b[j][3]), operand(s.a[2], s.a[3]), acc[j], 0, 0, 2, wb[j], 2, wa);
+  };
 #pragma unroll
-      for (int j = 0; j < CB; ++j) {
-        const uint32_t at = br[j] * 64 + 16 * half;
-        s.b[j][0] = load16(b0, at);
-        s.b[j][1] = load16(b0, at + 32);
-        s.b[j][2] = load16(b0 + b_chunk, at);
-        s.b[j][3] = load16(b0 + b_chunk, at + 32);
-        s.sb[j] = *reinterpret_cast<const uint32_t*>(bs0 + br[j] * 4);
-      }
-      const uint32_t at = ar * 64 + 16 * half;
-      s.a[0] = load16(a0, at);
-      s.a[1] = load16(a0, at + 32);
-      s.a[2] = load16(a0 + a_chunk, at);
-      s.a[3] = load16(a0 + a_chunk, at + 32);
-      s.sa = *reinterpret_cast<const uint32_t*>(as0 + ar * 4);
-    };
-    // Lane half h's scale byte is byte h of a word in its first step and 2 + h in its
-    // second: the word shifted by h bytes, the MFMA taking its byte 0, then 2.
-    auto multiply = [&](const Pair<CB>& s) {
-      const int wa = static_cast<int>(s.sa >> (8 * half));
-      int wb[CB];
-#pragma unroll
-      for (int j = 0; j < CB; ++j) wb[j] = static_cast<int>(s.sb[j] >> (8 * half));
-#pragma unroll
-      for (int j = 0; j < CB; ++j)
-        acc[j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-            operand(s.b[j][0], s.b[j][1]), operand(s.a[0], s.a[1]), acc[j], 0, 0, 0, wb[j], 0, wa);
-#pragma unroll
-      for (int j = 0; j < CB; ++j)
-        acc[j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-            operand(s.b[j][2], s.b[j][3]), operand(s.a[2], s.a[3]), acc[j], 0, 0, 2, wb[j], 2, wa);
-    };
-#pragma unroll
-    for (int i = 0; i < D; ++i)
-      if (i < pairs) load(in[i], i);
-    int32_t p = 0;
-    for (; p + 2 * D <= pairs; p += D) {
-#pragma unroll
-      for (int i = 0; i < D; ++i) {
-        multiply(in[i]);
-        __builtin_amdgcn_sched_barrier(0);
-        load(in[i], p + D + i);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    // the last D to 2 D - 1 pairs (all of them where there are fewer)
+  for (int i = 0; i < D; ++i)
+    if (i < pairs) load(in[i], i);
+  int32_t p = 0;
+  for (; p + 2 * D <= pairs; p += D) {
 #pragma unroll
     for (int i = 0; i < D; ++i) {
-      if (p + i < pairs) multiply(in[i]);
+      multiply(in[i]);
       __builtin_amdgcn_sched_barrier(0);
-      if (p + D + i < pairs) load(in[i], p + D + i);
+      load(in[i], p + D + i);
       __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int i = 0; i < D; ++i)
-      if (p + D + i < pairs) multiply(in[i]);
-
-    // lane l holds row l % 32, run g the columns 8 g + 4 (l / 32) .. + 3 of each block
-    const int32_t row = row0 + r32;
-    if (row >= t.lo + rows) continue;
-#pragma unroll
-    for (int j = 0; j < CB; ++j)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int32_t col = col0 + 32 * j + 8 * g + 4 * half;
-        if (col >= n) continue;  // n is a multiple of 4
-        T* at = y + static_cast<int64_t>(row) * n + col;
-        const float c[4] = {acc[j][4 * g], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]};
-        if constexpr (std::is_same<T, uint16_t>::value)
-          *reinterpret_cast<uint2*>(at) = make_uint2(pack_bf16x2(c[0], c[1]), pack_bf16x2(c[2], c[3]));
-        else
-          *reinterpret_cast<float4*>(at) = make_float4(c[0], c[1], c[2], c[3]);
-      }
   }
+  // the last D to 2 D - 1 pairs (all of them where there are fewer)
+#pragma unroll
+  for (int i = 0; i < D; ++i) {
+    if (p + i < pairs) multiply(in[i]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (p + D + i < pairs) load(in[i], p + D + i);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int i = 0; i < D; ++i)
+    if (p + D + i < pairs) multiply(in[i]);
+
+  // lane l holds row l % 32, run g the columns 8 g + 4 (l / 32) .. + 3 of each block
+  const int32_t row = row0 + r32;
+  if (row >= end) return;
+#pragma unroll
+  for (int j = 0; j < CB; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int32_t col = col0 + 32 * j + 8 * g + 4 * half;
+      if (col >= n) continue;  // n is a multiple of 4
+      T* at = y + static_cast<int64_t>(row) * n + col;
+      const float c[4] = {acc[j][4 * g], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]};
+      if constexpr (std::is_same<T, uint16_t>::value)
+        *reinterpret_cast<uint2*>(at) = make_uint2(pack_bf16x2(c[0], c[1]), pack_bf16x2(c[2], c[3]));
+      else
+        *reinterpret_cast<float4*>(at) = make_float4(c[0], c[1], c[2], c[3]);
+    }
 }
 
-template <typename T, int CB>
+template <typename T>
 int launch_as(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b_values,
               const uint8_t* b_scales, const void* list, int64_t slots, int32_t groups, int64_t m,
               int64_t n, int64_t k, int64_t height, void* y, hipStream_t s) {
-  const int64_t col_blocks = ceil_div(n, WAVES * 32 * CB);
+  const int64_t col_blocks = ceil_div(n, 32 * CB);
   if (slots * col_blocks >= (1LL << 31)) return fail(BUX_E_ARGUMENT, "bux_mx_grouped_rows: too many tiles");
-  hipLaunchKernelGGL((rows_direct_kernel<T, CB>), dim3(static_cast<unsigned>(slots * col_blocks)),
-                     dim3(THREADS), 0, s, a_values, a_scales, b_values, b_scales,
-                     static_cast<int32_t>(k), static_cast<int32_t>(m), static_cast<int32_t>(n), groups,
+  const int64_t rows = m > height ? m : height;  // no tile holds more
+  const int64_t row_blocks = ceil_div(rows < BM ? rows : BM, BLOCK);
+  hipLaunchKernelGGL(rows_direct_kernel<T>,
+                     dim3(static_cast<unsigned>(slots * col_blocks), static_cast<unsigned>(row_blocks)),
+                     dim3(64), 0, s, a_values, a_scales, b_values, b_scales, static_cast<int32_t>(k),
+                     static_cast<int32_t>(m), static_cast<int32_t>(n), groups,
                      static_cast<int32_t>(height), starts_in(list), tiles_in(list, groups),
                      static_cast<int32_t>(col_blocks), static_cast<T*>(y));
   return launched("rows_direct_kernel");
@@ -184,27 +182,27 @@ int launch_as(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b
 
 }  // namespace
 
-// The line between the two kernels, by the mean rows a group (the sizes are the device's).
-// Measured against grouped_mx.hip's on 128 groups, even routing (us): K 2048, N 1536, 64
-// rows 56 -> 37, 512 rows 85 -> 72, 1600 rows 83 -> 76, 2400 rows 87 -> 78, 3200 rows 87 ->
-// 100; K 768, N 2048: 28 -> 18, 52 -> 39, 52 -> 42, 53 -> 43, 52 -> 49. From 20 rows a group on,
-// groups past one block of 32 rows make waves read B's bytes again.
-bool rows_direct(int64_t m, int32_t groups) { return m > 0 && m <= 20 * static_cast<int64_t>(groups); }
+// The line between the two kernels, by the mean rows a group (the sizes are the device's)
+// and whether the tiled one's 256-column tiles fill half of the chip. Measured against
+// grouped_mx.hip's (us; even loads, then Zipf(1.2)): 128 groups of K 2048, N 1536, half a row
+// a group 53 -> 29, 28 -> 21; 6 rows 90 -> 73, 83 -> 67; 16 rows 88 -> 77, 87 -> 89; 26 rows 90
+// -> 93, 107 -> 106; 16 groups of K 6400, N 4096, 6 rows 90 -> 76, 89 -> 85; 16 rows 88 -> 78, 86
+// -> 96; 32 rows 86 -> 106. Few tiles: 8 groups of K 7168, N 4096, 12 rows 80 -> 44, 32 rows 80
+// -> 55; of K 2048, N 1536, 32 rows 27 -> 13.
+bool rows_direct(int64_t m, int32_t groups, int64_t n) {
+  const bool few = groups * ceil_div(n, BN) <= 128;
+  return m > 0 && m <= (few ? 32 : 16) * static_cast<int64_t>(groups);
+}
 
 int launch_rows_direct(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b_values,
                        const uint8_t* b_scales, const void* list, int64_t slots, int32_t groups,
                        int64_t m, int64_t n, int64_t k, int64_t height, int out_dtype, void* y,
                        hipStream_t s) {
-  // A wave takes 64 columns, half of A's reads a column that 32 take, once such waves
-  // fill the chip; about m groups / (m + groups) groups have a row. 128 groups of K 2048,
-  // N 1536 with 32 and with 64 columns a wave (us): 160 rows 57 and 61, 256 rows 66 and 67,
-  // 1600 rows 80 and 76.
-  const bool wide = m * groups / (m + groups) * ceil_div(n, 64) >= 2100;
-  auto go = [&](auto launch) {
-    return launch(a_values, a_scales, b_values, b_scales, list, slots, groups, m, n, k, height, y, s);
-  };
-  if (out_dtype == BUX_BF16) return wide ? go(launch_as<uint16_t, 2>) : go(launch_as<uint16_t, 1>);
-  return wide ? go(launch_as<float, 2>) : go(launch_as<float, 1>);
+  return out_dtype == BUX_BF16
+             ? launch_as<uint16_t>(a_values, a_scales, b_values, b_scales, list, slots, groups, m, n,
+                                   k, height, y, s)
+             : launch_as<float>(a_values, a_scales, b_values, b_scales, list, slots, groups, m, n, k,
+                                height, y, s);
 }
 
 }  // namespace bux
