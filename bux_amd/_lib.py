@@ -59,6 +59,8 @@ SIGNATURES = {
     "bux_version": (_int, []),
     "bux_moe_permute_workspace_size": (_size, [_i64, _i32]),
     "bux_moe_permute": (_int, [_p, _i64, _i32, _p, _p, _p, _p, _p, _size, _p]),
+    "bux_moe_permute_layer": (
+        _int, [_p, _i64, _i32, _p, _i32, _p, _p, _p, _p, _p, _p, _size, _i64, _i64, _p, _size, _p]),
     "bux_mx_quantize": (
         _int, [_p, _p, _i32, _i64, _i64, _i64, _i64, _i64, _p, _int, _p, _p, _p, _p, _p]),
     "bux_mx_quantize_f32": (

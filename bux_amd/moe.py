@@ -63,6 +63,37 @@ def sort_by_expert(idx: torch.Tensor, num_experts: int) -> Sorted:
     return Sorted(order, inverse, sizes, offsets)
 
 
+def sort_for_layer(
+    idx: torch.Tensor, num_experts: int, weights: torch.Tensor, height: int | None,
+) -> tuple[Sorted, torch.Tensor, grouped_mxfp8.TileList | None]:
+    """Return `sort_by_expert`, `picked_weights` of it and, with `height`, the MXFP8 GEMMs'
+    `tiles_of` its sizes (a of `height` rows, outputs of the picks), in the sort's own
+    kernels. weights: bfloat16 or float32, one a pick."""
+    n = idx.numel()
+    weights = weights.reshape(-1)
+    if weights.numel() != n:  # picks past the weights weigh 0
+        s = sort_by_expert(idx, num_experts)
+        listed = None if height is None else grouped_mxfp8.tiles_of(s.sizes, height, n)
+        return s, picked_weights(weights, s.order), listed
+    require(idx, weights)
+    if idx.dtype != torch.int32:
+        raise TypeError("idx is int32")
+    dev = idx.device
+    ints = torch.empty(2 * n + 2 * num_experts + 1, dtype=torch.int32, device=dev)
+    order, inverse, sizes, offsets = ints.split([n, n, num_experts, num_experts + 1])
+    row_weights = torch.empty(n, dtype=weights.dtype, device=dev)
+    buf = None
+    if height is not None:
+        buf = workspace(lib().bux_mx_grouped_rows_workspace_size(num_experts, height, n), dev)
+    ws = workspace(lib().bux_moe_permute_workspace_size(n, num_experts), dev)
+    _lib.check(lib().bux_moe_permute_layer(
+        ptr(idx), n, num_experts, ptr(weights), weights.element_size(), ptr(order), ptr(inverse),
+        ptr(sizes), ptr(offsets), ptr(row_weights), ptr(buf), 0 if buf is None else buf.numel(),
+        height or 0, n, ptr(ws), ws.numel(), stream()))
+    listed = None if buf is None else grouped_mxfp8.TileList(buf, num_experts, height, n)
+    return Sorted(order, inverse, sizes, offsets), row_weights, listed
+
+
 def token_rows(z: torch.Tensor, order: torch.Tensor, k: int) -> torch.Tensor:
     """Return ``z[order // k]`` (bfloat16 or float32 rows), a row of 0 where ``order //
     k`` lies outside z's rows (a negative entry too; the sort's orders never do)."""
@@ -569,20 +600,17 @@ def experts_forward(
         fused = False  # the fused up GEMM's epilogue is bfloat16's
     if quantized is not None:
         quantized.check(fmt, up, down)
+    height = grouped_mxfp8.whole(m)
     with span("permute"):
-        s = sort_by_expert(idx, e)
+        # with one tile list for the step's six GEMMs: a of `height` rows, outputs of m
+        s, row_weights, listed = sort_for_layer(idx, e, weights,
+                                                height if fprop or dgrad or wgrad else None)
         filled = s.filled
-        row_weights = picked_weights(weights, s.order)
     up2 = up.reshape(e, d, f * p)
     tiles = fmt == "mxfp8_2d"
     # with a norm, the activation is not weighted: the norm's output is (moe.py:871)
     act_weights = row_weights if norm is None else torch.ones_like(row_weights)
-    height = grouped_mxfp8.whole(m)
-    x_k = x_m = up_n = up_k = h_k = h_m = down_n = down_k = rows = listed = None
-    if fprop or dgrad or wgrad:
-        with span("tile list"):
-            # one tile list for the step's six GEMMs: a of `height` rows, outputs of m
-            listed = grouped_mxfp8.tiles_of(s.sizes, height, m)
+    x_k = x_m = up_n = up_k = h_k = h_m = down_n = down_k = rows = None
     if fprop or wgrad:
         with span("quantize x"):
             # the copies its passes take (grouped_blockscaled.py:180-183): x along k for

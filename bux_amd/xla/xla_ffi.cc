@@ -102,6 +102,23 @@ XLA_FFI_DEFINE_HANDLER_SYMBOL(BuxMoePermute, MoePermute,
                               ffi::Ffi::Bind().Ctx<Stream>().Arg<In>().Attr<int64_t>("num_experts")
                                   .Ret<In>().Ret<In>().Ret<In>().Ret<In>().Ret<In>());
 
+// weights: one a pick, bfloat16 or float32; list: bux_mx_grouped_tiles's buffer, or empty.
+static ffi::Error MoePermuteLayer(hipStream_t s, In idx, In weights, int64_t num_experts,
+                                  int64_t m, int64_t height, Out order, Out inverse, Out sizes,
+                                  Out offsets, Out row_weights, Out list, Out ws) {
+  return status(bux_moe_permute_layer(
+      at<const int32_t>(idx), static_cast<int64_t>(idx.element_count()),
+      static_cast<int32_t>(num_experts), at<const void>(weights),
+      f32(weights) ? 4 : 2, at<int32_t>(order), at<int32_t>(inverse),
+      at<int32_t>(sizes), at<int32_t>(offsets), at<void>(row_weights), at<void>(list),
+      list->size_bytes(), m, height, at<void>(ws), ws->size_bytes(), s));
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(BuxMoePermuteLayer, MoePermuteLayer,
+                              ffi::Ffi::Bind().Ctx<Stream>().Arg<In>().Arg<In>()
+                                  .Attr<int64_t>("num_experts").Attr<int64_t>("m")
+                                  .Attr<int64_t>("height").Ret<In>().Ret<In>().Ret<In>().Ret<In>()
+                                  .Ret<In>().Ret<In>().Ret<In>());
+
 // --- a-4: MXFP8 quantization -----------------------------------------------------------
 
 // x [groups, rows, cols] (or with an index the matrix read from), bfloat16 or float32;

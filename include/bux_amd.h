@@ -74,6 +74,20 @@ size_t bux_moe_permute_workspace_size(int64_t n_picks, int32_t num_experts);
 int bux_moe_permute(const int32_t* idx, int64_t n_picks, int32_t num_experts, int32_t* order,
                     int32_t* inverse, int32_t* sizes, int32_t* offsets, void* workspace,
                     size_t workspace_bytes, void* stream);
+/* bux_moe_permute_layer: the same sort with what the layer makes of it, in the same
+ * kernels (routed's picked_weights, experts/moe.py:766-767, and the GEMMs' tiles_of):
+ *
+ * weights      n_picks words of `weight_bytes` (2 or 4), each pick's weight.
+ * row_weights  n_picks words: weights[order[i]].
+ * list         NULL, or the tile list bux_mx_grouped_tiles makes of the sizes for m and
+ *              height (num_experts up to its limit; the larger of m and height at least
+ *              n_picks), list_bytes as bux_mx_grouped_rows_workspace_size gives. */
+int bux_moe_permute_layer(const int32_t* idx, int64_t n_picks, int32_t num_experts,
+                          const void* weights, int32_t weight_bytes, int32_t* order,
+                          int32_t* inverse, int32_t* sizes, int32_t* offsets, void* row_weights,
+                          void* list, size_t list_bytes, int64_t m, int64_t height,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
 
 /* ---------------------------------------------------------------------------------
  * a-4. MXFP8 quantization of a matrix and of its transpose, in one pass.

@@ -361,3 +361,18 @@ def test_each_xla_ffi_handler_passes_every_argument_the_header_declares():
     for name, counts in calls.items():
         assert name in declared, name
         assert set(counts) == {declared[name]}, (name, counts, declared[name])
+
+
+def test_the_layers_sort_rejects_bad_arguments(lib):
+    p = ctypes.c_void_p(16)
+
+    def sort(n=100, e=8, word=2, list_bytes=1 << 20, m=128, height=100, ws=1 << 20, weights=p):
+        return lib.bux_moe_permute_layer(p, n, e, weights, word, p, p, p, p, p, p, list_bytes, m, height,
+                                         p, ws, None)
+
+    assert sort(word=8) == 1 and "weight_bytes=8" in _msg(lib)
+    assert sort(weights=None) == 1 and "weights" in _msg(lib)
+    assert sort(e=0) == 1 and "groups=0" in _msg(lib)
+    assert sort(m=64, height=96) == 1 and "100 picks" in _msg(lib)  # a list shorter than the picks
+    assert sort(list_bytes=64) == 2 and "list" in _msg(lib)
+    assert sort(ws=4) == 2 and "workspace" in _msg(lib)
