@@ -18,10 +18,18 @@
 // groups: the picks outside the experts, whose weights the layer zeroes) give 0.
 //
 // Forward: a workgroup a row, the row in registers (d <= 8192: 8 values a thread a 2048
-// chunk), block sums through LDS. Backward: a workgroup takes ROWS rows one after another,
-// each thread the same columns of every row, so that it adds its columns' gain and bias
-// gradients over the rows in registers; one float32 partial a workgroup and column goes
-// to the workspace, and norm_params_kernel adds the partials in workgroup order.
+// chunk), block sums through LDS. Backward: a workgroup takes rows_a_block rows one after
+// another, each thread the same columns of every row, so that it adds its columns' gain and
+// bias gradients over the rows in registers; one float32 partial a workgroup and column
+// goes to the workspace, and norm_params_kernel adds the partials in a fixed order.
+//
+// Both are bound by a row's chain of loads and block sums (about 4 us a row backward), so
+// what counts is the rows in flight: the chunks are a template parameter, which keeps the
+// registers of a narrow row (d 1024: 188 -> 60) from holding four workgroups' worth of a
+// CU, and a backward workgroup takes few rows where there are few (64 each put 4004 rows
+// on 63 CUs: 259 us in float32 at d 1024, and 19 us for the partials; now 25 and 9).
+
+#include <type_traits>
 
 #include "common.h"
 #include "glu.h"
@@ -32,7 +40,13 @@ namespace {
 constexpr int THREADS = 256;
 constexpr int VEC = 8;
 constexpr int MAX_CHUNKS = 4;  // d <= MAX_CHUNKS * THREADS * VEC = 8192
-constexpr int ROWS = 64;       // rows a backward workgroup
+constexpr int MAX_ROWS = 64;   // rows a backward workgroup, at most
+
+// The rows a backward workgroup takes of m: about 1024 workgroups (4 a CU).
+int64_t rows_a_block(int64_t m) {
+  const int64_t r = (m + 1023) / 1024;
+  return r < 1 ? 1 : (r < MAX_ROWS ? r : MAX_ROWS);
+}
 
 // The sum of v over the workgroup (256 threads); `red` 4 floats of LDS. Every thread
 // gets it; the LDS is free again when it returns.
@@ -60,21 +74,22 @@ struct NormArgs {
   int32_t experts;
 };
 
-// One thread's share of a row: columns c(i) = (i * THREADS + threadIdx.x) * VEC + j.
+// One thread's share of a row of C chunks: columns c(i) = (i * THREADS + threadIdx.x) * VEC + j.
+template <int C>
 struct Row {
-  float v[MAX_CHUNKS][VEC];
+  float v[C][VEC];
 };
 
 // The row's values through the norm's input side: y + down bias, rounded; with
 // scale_input, times the gain, rounded (`in` before it, `x` after). Columns past d: 0.
-template <typename T>
+template <int C, typename T>
 __device__ __forceinline__ void norm_input(const NormArgs<T>& a, const T* y_row, int32_t e,
-                                           int64_t d, Row& in, Row& x, Row& gain) {
+                                           int64_t d, Row<C>& in, Row<C>& x, Row<C>& gain) {
   // Each product rounds before it is added, as the reference's ops do (no FMA contraction).
 #pragma clang fp contract(off)
   using E = Elem<T>;
 #pragma unroll
-  for (int i = 0; i < MAX_CHUNKS; ++i) {  // every chunk: past d, zeros
+  for (int i = 0; i < C; ++i) {  // columns past d: zeros
     const int64_t c = (static_cast<int64_t>(i) * THREADS + threadIdx.x) * VEC;
     float yv[VEC] = {0, 0, 0, 0, 0, 0, 0, 0}, b[VEC] = {0, 0, 0, 0, 0, 0, 0, 0};
     float s[VEC] = {1, 1, 1, 1, 1, 1, 1, 1};
@@ -95,24 +110,23 @@ __device__ __forceinline__ void norm_input(const NormArgs<T>& a, const T* y_row,
 }
 
 // mean (layernorm, else 0) and rsqrt(mean((x - mean)^2) + eps) of the row, float32.
-template <typename T>
-__device__ __forceinline__ void norm_stats(const NormArgs<T>& a, const Row& x, int64_t d, int chunks,
-                                           float* red, float* mean, float* rs) {
+template <int C, typename T>
+__device__ __forceinline__ void norm_stats(const NormArgs<T>& a, const Row<C>& x, int64_t d, float* red,
+                                           float* mean, float* rs) {
   // Each product rounds before it is added, as the reference's ops do (no FMA contraction).
 #pragma clang fp contract(off)
   float m = 0.0f;
   if (a.kind == BUX_LAYERNORM) {
     float t = 0.0f;
 #pragma unroll
-    for (int i = 0; i < MAX_CHUNKS; ++i)
+    for (int i = 0; i < C; ++i)
 #pragma unroll
       for (int j = 0; j < VEC; ++j) t += x.v[i][j];  // columns past d hold 0
     m = block_sum(t, red) / static_cast<float>(d);
   }
   float q = 0.0f;
 #pragma unroll
-  for (int i = 0; i < MAX_CHUNKS; ++i) {
-    if (i >= chunks) break;
+  for (int i = 0; i < C; ++i) {
     const int64_t c = (static_cast<int64_t>(i) * THREADS + threadIdx.x) * VEC;
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
@@ -124,7 +138,7 @@ __device__ __forceinline__ void norm_stats(const NormArgs<T>& a, const Row& x, i
   *rs = rsqrtf(block_sum(q, red) / static_cast<float>(d) + a.eps);
 }
 
-template <typename T>
+template <typename T, int C>
 __global__ __launch_bounds__(THREADS) void norm_forward_kernel(
     const T* __restrict__ y, int64_t d, NormArgs<T> a, const T* __restrict__ weights,
     T* __restrict__ out) {
@@ -133,27 +147,24 @@ __global__ __launch_bounds__(THREADS) void norm_forward_kernel(
   using E = Elem<T>;
   __shared__ float red[4];
   const int64_t r = blockIdx.x;
-  const int chunks = static_cast<int>((d + THREADS * VEC - 1) / (THREADS * VEC));
   const int32_t e = expert_of(a.offsets, a.experts, r);
   T* o = out + r * d;
   if (e < 0) {  // a row in no expert: 0 (a uniform branch: the whole workgroup's row)
     const float z[VEC] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-    for (int i = 0; i < MAX_CHUNKS; ++i) {
-      if (i >= chunks) break;
+    for (int i = 0; i < C; ++i) {
       const int64_t c = (static_cast<int64_t>(i) * THREADS + threadIdx.x) * VEC;
       if (c < d) E::store8(o + c, z);
     }
     return;
   }
-  Row in, x, gain;
+  Row<C> in, x, gain;
   norm_input(a, y + r * d, e, d, in, x, gain);
   float mean, rs;
-  norm_stats(a, x, d, chunks, red, &mean, &rs);
+  norm_stats(a, x, d, red, &mean, &rs);
   const float w = E::value(weights[r]);
 #pragma unroll
-  for (int i = 0; i < MAX_CHUNKS; ++i) {
-    if (i >= chunks) break;
+  for (int i = 0; i < C; ++i) {
     const int64_t c = (static_cast<int64_t>(i) * THREADS + threadIdx.x) * VEC;
     if (c >= d) continue;
     float b[VEC] = {0, 0, 0, 0, 0, 0, 0, 0}, v[VEC];
@@ -169,43 +180,41 @@ __global__ __launch_bounds__(THREADS) void norm_forward_kernel(
   }
 }
 
-// A workgroup takes rows [blockIdx.x ROWS, + ROWS): dv and the weights' gradient a row,
+// A workgroup takes rows [blockIdx.x rows, + rows): dv and the weights' gradient a row,
 // and its columns' gain and bias gradients summed over its rows into partials[2][block][d].
-template <typename T>
+template <typename T, int C>
 __global__ __launch_bounds__(THREADS) void norm_backward_kernel(
     const T* __restrict__ dy, const int32_t* __restrict__ index, int32_t index_div,
-    int64_t sources, const T* __restrict__ y, int64_t m, int64_t d, NormArgs<T> a,
+    int64_t sources, const T* __restrict__ y, int64_t m, int64_t d, int64_t rows, NormArgs<T> a,
     const T* __restrict__ weights, T* __restrict__ dv, T* __restrict__ d_weights,
     float* __restrict__ partials) {
   // Each product rounds before it is added, as the reference's ops do (no FMA contraction).
 #pragma clang fp contract(off)
   using E = Elem<T>;
   __shared__ float red[4];
-  const int chunks = static_cast<int>((d + THREADS * VEC - 1) / (THREADS * VEC));
-  Row d_gain, d_bias;
+  Row<C> d_gain, d_bias;
 #pragma unroll
-  for (int i = 0; i < MAX_CHUNKS; ++i)
+  for (int i = 0; i < C; ++i)
 #pragma unroll
     for (int j = 0; j < VEC; ++j) d_gain.v[i][j] = d_bias.v[i][j] = 0.0f;
-  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * ROWS;
-  for (int64_t r = r0; r < r0 + ROWS && r < m; ++r) {
+  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rows;
+  for (int64_t r = r0; r < r0 + rows && r < m; ++r) {
     const int32_t e = expert_of(a.offsets, a.experts, r);
     T* o = dv + r * d;
     if (e < 0) {  // uniform: the whole workgroup's row
       const float z[VEC] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-      for (int i = 0; i < MAX_CHUNKS; ++i) {
-        if (i >= chunks) break;
+      for (int i = 0; i < C; ++i) {
         const int64_t c = (static_cast<int64_t>(i) * THREADS + threadIdx.x) * VEC;
         if (c < d) E::store8(o + c, z);
       }
       if (threadIdx.x == 0) d_weights[r] = E::make(0.0f);
       continue;
     }
-    Row in, x, gain;
+    Row<C> in, x, gain;
     norm_input(a, y + r * d, e, d, in, x, gain);
     float mean, rs;
-    norm_stats(a, x, d, chunks, red, &mean, &rs);
+    norm_stats(a, x, d, red, &mean, &rs);
     const float w = E::value(weights[r]);
     // dy's row: r, or by index (a row of 0 where that lies outside dy's sources rows)
     const int64_t src =
@@ -214,11 +223,10 @@ __global__ __launch_bounds__(THREADS) void norm_backward_kernel(
     const T* g_row = dy + (g_live ? src : 0) * d;
     // dn = g w; the weight's gradient sum_c g n (products rounded, as T's ops);
     // dxn = dn (times the gain); and the two sums the normalization's VJP takes
-    Row dxn;
+    Row<C> dxn;
     float wsum = 0.0f, s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
-    for (int i = 0; i < MAX_CHUNKS; ++i) {
-      if (i >= chunks) break;
+    for (int i = 0; i < C; ++i) {
       const int64_t c = (static_cast<int64_t>(i) * THREADS + threadIdx.x) * VEC;
       float g[VEC] = {0, 0, 0, 0, 0, 0, 0, 0}, b[VEC] = {0, 0, 0, 0, 0, 0, 0, 0};
       if (c < d) {
@@ -251,8 +259,7 @@ __global__ __launch_bounds__(THREADS) void norm_backward_kernel(
     const float mean_dxu = block_sum(s2, red) / static_cast<float>(d);
     if (threadIdx.x == 0) d_weights[r] = E::make(sum_w);
 #pragma unroll
-    for (int i = 0; i < MAX_CHUNKS; ++i) {
-      if (i >= chunks) break;
+    for (int i = 0; i < C; ++i) {
       const int64_t c = (static_cast<int64_t>(i) * THREADS + threadIdx.x) * VEC;
       if (c >= d) continue;
       float out[VEC];
@@ -274,8 +281,7 @@ __global__ __launch_bounds__(THREADS) void norm_backward_kernel(
   float* pg = partials + static_cast<int64_t>(blockIdx.x) * d;
   float* pb = partials + (static_cast<int64_t>(gridDim.x) + blockIdx.x) * d;
 #pragma unroll
-  for (int i = 0; i < MAX_CHUNKS; ++i) {
-    if (i >= chunks) break;
+  for (int i = 0; i < C; ++i) {
     const int64_t c = (static_cast<int64_t>(i) * THREADS + threadIdx.x) * VEC;
     if (c >= d) continue;
 #pragma unroll
@@ -286,20 +292,41 @@ __global__ __launch_bounds__(THREADS) void norm_backward_kernel(
   }
 }
 
-// d_gain[c] and d_bias[c]: the workgroups' partials added in workgroup order.
-__global__ __launch_bounds__(THREADS) void norm_params_kernel(const float* __restrict__ partials,
-                                                              int64_t blocks, int64_t d,
-                                                              float* __restrict__ d_gain,
-                                                              float* __restrict__ d_bias) {
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * THREADS + threadIdx.x;
-  if (c >= d) return;
+// d_gain[c] and d_bias[c]: the workgroups' partials, a workgroup 64 columns: its 16 waves
+// add every 16th partial in order, then the waves' sums in wave order.
+constexpr int PARAM_THREADS = 1024;
+__global__ __launch_bounds__(PARAM_THREADS) void norm_params_kernel(
+    const float* __restrict__ partials, int64_t blocks, int64_t d, float* __restrict__ d_gain,
+    float* __restrict__ d_bias) {
+  constexpr int WAVES = PARAM_THREADS / 64;
+  __shared__ float part[2][WAVES][64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t c = static_cast<int64_t>(blockIdx.x) * 64 + lane;
   float g = 0.0f, b = 0.0f;
-  for (int64_t k = 0; k < blocks; ++k) {
-    g += partials[k * d + c];
-    b += partials[(blocks + k) * d + c];
+  if (c < d) {
+#pragma unroll 8
+    for (int64_t k = wave; k < blocks; k += WAVES) {
+      g += partials[k * d + c];
+      b += partials[(blocks + k) * d + c];
+    }
   }
-  if (d_gain) d_gain[c] = g;
-  if (d_bias) d_bias[c] = b;
+  part[0][wave][lane] = g;
+  part[1][wave][lane] = b;
+  __syncthreads();
+  if (wave > 1 || c >= d) return;
+  float sum = part[wave][0][lane];
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w) sum += part[wave][w][lane];
+  float* out = wave == 0 ? d_gain : d_bias;
+  if (out) out[c] = sum;
+}
+
+// Calls f(std::integral_constant<int, C>{}) for a row of d columns in C chunks.
+template <typename F>
+void with_chunks(int64_t d, F&& f) {
+  if (d <= THREADS * VEC) f(std::integral_constant<int, 1>{});
+  else if (d <= 2 * THREADS * VEC) f(std::integral_constant<int, 2>{});
+  else f(std::integral_constant<int, MAX_CHUNKS>{});
 }
 
 template <typename T>
@@ -335,13 +362,15 @@ int norm_forward(const char* name, const T* y, int64_t m, int64_t d, const T* do
   if (int rc = norm_args(name, norm, scale, bias, down_bias, offsets, experts, &a)) return rc;
   if (m == 0) return BUX_OK;
   BUX_CHECK(y && weights && out, "%s: NULL buffer", name);
-  hipLaunchKernelGGL(norm_forward_kernel<T>, dim3(static_cast<unsigned>(m)), dim3(THREADS), 0,
-                     as_stream(stream), y, d, a, weights, out);
+  with_chunks(d, [&](auto c) {
+    hipLaunchKernelGGL((norm_forward_kernel<T, decltype(c)::value>), dim3(static_cast<unsigned>(m)),
+                       dim3(THREADS), 0, as_stream(stream), y, d, a, weights, out);
+  });
   return launched("norm_forward_kernel");
 }
 
 size_t backward_workspace(int64_t m, int64_t d) {
-  return static_cast<size_t>(2 * ceil_div(m, ROWS) * d) * sizeof(float);
+  return static_cast<size_t>(2 * ceil_div(m, rows_a_block(m)) * d) * sizeof(float);
 }
 
 template <typename T>
@@ -362,18 +391,21 @@ int norm_backward(const char* name, const T* dy, const int32_t* index, int32_t i
     return fail(BUX_E_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", name, workspace_bytes,
                 need);
   hipStream_t s = as_stream(stream);
-  const int64_t blocks = ceil_div(m, ROWS);
+  const int64_t rows = rows_a_block(m), blocks = ceil_div(m, rows);
   if (m > 0) {
     BUX_CHECK(dy && y && weights && dv && d_weights, "%s: NULL buffer", name);
-    hipLaunchKernelGGL(norm_backward_kernel<T>, dim3(static_cast<unsigned>(blocks)), dim3(THREADS),
-                       0, s, dy, index, index_div, sources, y, m, d, a, weights, dv, d_weights,
-                       static_cast<float*>(workspace));
+    with_chunks(d, [&](auto c) {
+      hipLaunchKernelGGL((norm_backward_kernel<T, decltype(c)::value>),
+                         dim3(static_cast<unsigned>(blocks)), dim3(THREADS), 0, s, dy, index,
+                         index_div, sources, y, m, d, rows, a, weights, dv, d_weights,
+                         static_cast<float*>(workspace));
+    });
     if (int rc = launched("norm_backward_kernel")) return rc;
   }
   if (!a.affine && !a.biased) return BUX_OK;
   // with no rows, the sums are 0: a workspace of no partials
-  hipLaunchKernelGGL(norm_params_kernel, dim3(static_cast<unsigned>(ceil_div(d, THREADS))),
-                     dim3(THREADS), 0, s, static_cast<const float*>(workspace), blocks, d,
+  hipLaunchKernelGGL(norm_params_kernel, dim3(static_cast<unsigned>(ceil_div(d, 64))),
+                     dim3(PARAM_THREADS), 0, s, static_cast<const float*>(workspace), blocks, d,
                      a.affine ? d_scale : nullptr, a.biased ? d_bias : nullptr);
   return launched("norm_params_kernel");
 }

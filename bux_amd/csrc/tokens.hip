@@ -359,54 +359,64 @@ __global__ __launch_bounds__(THREADS) void expert_bias_add_kernel(
 }
 
 // out[e] = sum over e's rows of v_r (x[src(r)], times weights[r] rounded to T if
-// weights). Workgroup (e, column chunk): wave w adds rows w, w + 4, ... of e in order,
-// lanes 8 columns each; the four waves' sums are added in wave order. Deterministic.
-constexpr int SUM_COLS = 64 * VEC;  // a workgroup's columns
+// weights). Workgroup (e, 256 columns): its 16 waves add every 16th row of e in order, four
+// rows' loads in flight and lanes 4 columns each; the waves' sums are added in wave order.
+// Deterministic. What bounds it is the rows a wave adds one after another: 16 experts of
+// 250 rows of 1024 float32 took 28 us by 4 waves of 512 columns (32 workgroups), now 6.5.
+constexpr int SUM_THREADS = 1024;
+constexpr int SUM_VEC = 4;
+constexpr int SUM_COLS = 64 * SUM_VEC;  // a workgroup's columns
 template <typename T>
-__global__ __launch_bounds__(THREADS) void expert_sums_kernel(
+__global__ __launch_bounds__(SUM_THREADS) void expert_sums_kernel(
     const T* __restrict__ x, const int32_t* __restrict__ index, int32_t index_div,
     int64_t sources, const T* __restrict__ weights, int64_t m, int64_t width,
     const int32_t* __restrict__ offsets, int32_t experts, float* __restrict__ out) {
   // Each product rounds before it is added, as the reference's ops do (no FMA contraction).
 #pragma clang fp contract(off)
   using E = Elem<T>;
-  __shared__ float part[THREADS / 64][SUM_COLS];
+  constexpr int WAVES = SUM_THREADS / 64, AT_ONCE = 4;
+  __shared__ float part[WAVES][SUM_COLS];
   const int64_t chunks = (width + SUM_COLS - 1) / SUM_COLS;
   const int64_t e = blockIdx.x / chunks;
   const int64_t c0 = (blockIdx.x % chunks) * SUM_COLS;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t c = c0 + lane * VEC;
+  const int64_t c = c0 + lane * SUM_VEC;
   // rows inside [0, m) only, whatever the offsets say
   const int64_t lo = offsets[e] > 0 ? offsets[e] : 0;
   const int64_t hi = offsets[e + 1] < m ? offsets[e + 1] : m;
-  float acc[VEC] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (c < width) {
-    for (int64_t r = lo + wave; r < hi; r += THREADS / 64) {
-      const int64_t src = index ? source_row(index[r], index_div, sources) : r;
-      if (src < 0) continue;  // a row of 0
-      float v[VEC];
-      E::load8(x + src * width + c, v);
-      if (weights) {
-        const float w = E::value(weights[r]);
+  float acc[SUM_VEC] = {0, 0, 0, 0};
+  if (c < width) {  // width is a multiple of 8: a lane's columns are all in or out
+    for (int64_t r0 = lo + wave; r0 < hi; r0 += WAVES * AT_ONCE) {
+      float v[AT_ONCE][SUM_VEC];
+      bool live[AT_ONCE];
 #pragma unroll
-        for (int q = 0; q < VEC; ++q) v[q] = E::round(v[q] * w);
+      for (int i = 0; i < AT_ONCE; ++i) {
+        const int64_t r = r0 + WAVES * i;
+        const int64_t src = r >= hi ? -1 : (index ? source_row(index[r], index_div, sources) : r);
+        live[i] = src >= 0;  // else past the rows, or a row of 0
+        if (!live[i]) continue;
+        load4(x + src * width + c, v[i]);
+        if (weights) {
+          const float w = E::value(weights[r]);
+#pragma unroll
+          for (int q = 0; q < SUM_VEC; ++q) v[i][q] = E::round(v[i][q] * w);
+        }
       }
 #pragma unroll
-      for (int q = 0; q < VEC; ++q) acc[q] += v[q];
+      for (int i = 0; i < AT_ONCE; ++i)
+#pragma unroll
+        for (int q = 0; q < SUM_VEC; ++q) acc[q] = live[i] ? acc[q] + v[i][q] : acc[q];
     }
   }
 #pragma unroll
-  for (int q = 0; q < VEC; ++q) part[wave][lane * VEC + q] = acc[q];
+  for (int q = 0; q < SUM_VEC; ++q) part[wave][lane * SUM_VEC + q] = acc[q];
   __syncthreads();
-  // thread t: column t and t + 256 of the chunk
-  for (int j = threadIdx.x; j < SUM_COLS; j += THREADS) {
-    const int64_t col = c0 + j;
-    if (col >= width) continue;
-    float sum = part[0][j];
+  const int j = threadIdx.x;  // a thread a column
+  if (j >= SUM_COLS || c0 + j >= width) return;
+  float sum = part[0][j];
 #pragma unroll
-    for (int w = 1; w < THREADS / 64; ++w) sum += part[w][j];
-    out[e * width + col] = sum;
-  }
+  for (int w = 1; w < WAVES; ++w) sum += part[w][j];
+  out[e * width + c0 + j] = sum;
 }
 
 // d_weights[r] += sum_c dy[src(r)][c] bias[e(r)][c]: one wave a row, lanes 8 columns a
@@ -556,7 +566,7 @@ int expert_sums(const char* name, const T* x, const int32_t* index, int32_t inde
   const int64_t chunks = ceil_div(width, SUM_COLS);
   BUX_CHECK(experts * chunks < (1LL << 31), "%s: too large", name);
   hipLaunchKernelGGL(expert_sums_kernel<T>, dim3(static_cast<unsigned>(experts * chunks)),
-                     dim3(THREADS), 0, as_stream(stream), x, index, index_div, sources, weights,
+                     dim3(SUM_THREADS), 0, as_stream(stream), x, index, index_div, sources, weights,
                      m, width, offsets, experts, out);
   return launched("expert_sums_kernel");
 }
