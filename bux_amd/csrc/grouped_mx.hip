@@ -389,8 +389,8 @@ __device__ __forceinline__ void stream8(void* at, uint32_t x, uint32_t y) {
 // this way 627.) I, J: the wave's blocks of 32 rows and columns, its first row and column
 // row0 and col0 of the tile; the rows [0, rows) and columns [0, cols) are stored (cols a
 // multiple of 4).
-template <int I, int J>
-__device__ void store_f32(const v16f acc[4][4], float* tile, int32_t ld, int32_t rows, int32_t cols,
+template <int I, int J, typename Values>
+__device__ void store_f32(const Values& values, float* tile, int32_t ld, int32_t rows, int32_t cols,
                           int32_t row0, int32_t col0, Stage& stage) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   constexpr int FP = 272;
@@ -405,11 +405,8 @@ __device__ void store_f32(const v16f acc[4][4], float* tile, int32_t ld, int32_t
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const v16f& a = acc[i][jj + b];
-          *reinterpret_cast<float4*>(mine + b * 128 + g * 32) =
-              make_float4(a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]);
-        }
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<float4*>(mine + b * 128 + g * 32) = values.f32(i, jj + b, g);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_wave_barrier();
       uint4 v[8];
@@ -440,15 +437,44 @@ static_assert(4 * 32 * PITCH == sizeof(Stage), "the epilogue's regions fill a st
 // With LO, only the rows from row_lo on are stored.
 // The accumulators of a 32 x 32 block as bfloat16 pairs: run g's columns 0-1 and 2-3
 // (v_cvt_pk_bf16_f32: two floats to two bfloat16, nearest even).
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
+}
 struct FromAcc {
   const v16f (*acc)[4];
   __device__ __forceinline__ uint2 operator()(int i, int j, int g) const {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
     const v16f& a = acc[i][j];
-    const bf16x2 lo = __builtin_convertvector((f32x2{a[4 * g], a[4 * g + 1]}), bf16x2);
-    const bf16x2 hi = __builtin_convertvector((f32x2{a[4 * g + 2], a[4 * g + 3]}), bf16x2);
-    return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+    return make_uint2(bf16_pair(a[4 * g], a[4 * g + 1]), bf16_pair(a[4 * g + 2], a[4 * g + 3]));
+  }
+  __device__ __forceinline__ float4 f32(int i, int j, int g) const {
+    const v16f& a = acc[i][j];
+    return make_float4(a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]);
+  }
+};
+
+// FromAcc's values with their column's bias added as an op of its own does: the product
+// rounded to the output's type, then the sum. A tile holds one group's rows, so a lane's
+// biases are those of its columns, 4 a run: read once a tile, before the stores.
+struct FromAccBiased16 {
+  FromAcc from;
+  uint2 bias[4][4];
+  __device__ __forceinline__ static uint32_t add(uint32_t x, uint32_t y) {
+    return bf16_pair(__uint_as_float(x << 16) + __uint_as_float(y << 16),
+                     __uint_as_float(x & 0xffff0000u) + __uint_as_float(y & 0xffff0000u));
+  }
+  __device__ __forceinline__ uint2 operator()(int i, int j, int g) const {
+    const uint2 v = from(i, j, g);
+    return make_uint2(add(v.x, bias[j][g].x), add(v.y, bias[j][g].y));
+  }
+};
+struct FromAccBiased32 {
+  FromAcc from;
+  float4 bias[4][4];
+  __device__ __forceinline__ float4 f32(int i, int j, int g) const {
+    const float4 v = from.f32(i, j, g), b = bias[j][g];
+    return make_float4(v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w);
   }
 };
 
@@ -507,22 +533,24 @@ __device__ void store_bf16(const Pairs& pairs, uint16_t* tile, int32_t ld, int32
   }
 }
 
-__device__ __forceinline__ void store_tile(const v16f acc[4][4], uint16_t* tile, int32_t ld,
+template <typename From>
+__device__ __forceinline__ void store_tile(const From& from, uint16_t* tile, int32_t ld,
                                            int32_t rows, int32_t cols, Stage& stage) {
-  store_bf16(FromAcc{acc}, tile, ld, rows, cols, stage);
+  store_bf16(from, tile, ld, rows, cols, stage);
 }
-__device__ __forceinline__ void store_tile(const v16f acc[4][4], float* tile, int32_t ld,
+template <typename From>
+__device__ __forceinline__ void store_tile(const From& from, float* tile, int32_t ld,
                                            int32_t rows, int32_t cols, Stage& stage) {
   const int wave = threadIdx.x >> 6;
-  store_f32<4, 4>(acc, tile, ld, rows, cols, (wave >> 1) * 128, (wave & 1) * 128, stage);
+  store_f32<4, 4>(from, tile, ld, rows, cols, (wave >> 1) * 128, (wave & 1) * 128, stage);
 }
 
 // A half tile's outputs, each wave's 128 rows x 64 columns (columns 64 w on; accumulator
 // blocks [i][0..1]). bfloat16 through the wave's region of the stage as store_bf16 does,
 // read back 16 bytes a lane, 8 lanes a row, in 4 rounds of 32 rows.
-__device__ void store_tile_half(const v16f acc[4][4], uint16_t* tile, int32_t ld, int32_t rows,
+template <typename From>
+__device__ void store_tile_half(const From& pairs, uint16_t* tile, int32_t ld, int32_t rows,
                                 int32_t cols, Stage& stage) {
-  const FromAcc pairs{acc};
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint8_t* region = reinterpret_cast<uint8_t*>(&stage) + wave * 32 * PITCH;
   uint8_t* mine = region + (lane & 31) * PITCH + 8 * (lane >> 5);
@@ -566,10 +594,11 @@ __device__ void store_tile_half(const v16f acc[4][4], uint16_t* tile, int32_t ld
   }
 }
 // float32 as store_f32.
-__device__ void store_tile_half(const v16f acc[4][4], float* tile, int32_t ld, int32_t rows,
+template <typename From>
+__device__ void store_tile_half(const From& from, float* tile, int32_t ld, int32_t rows,
                                 int32_t cols, Stage& stage) {
   const int wave = threadIdx.x >> 6;
-  store_f32<4, 2>(acc, tile, ld, rows, cols, 0, wave * 64, stage);
+  store_f32<4, 2>(from, tile, ld, rows, cols, 0, wave * 64, stage);
 }
 
 // bfloat16 of a tile that stores every row and column (PH: a half tile's 128 rows),
@@ -587,8 +616,8 @@ constexpr int PAIR_PITCH = 136;
 constexpr int PAIR_BUF = 32 * PAIR_PITCH;
 static_assert(2 * PAIR_BUF == 32 * PITCH, "a wave's two pair buffers fill its region of the stage");
 
-template <bool PH>
-__device__ void store_pairs(const v16f acc[4][4], uint16_t* tile, int32_t ld, Stage& stage) {
+template <bool PH, typename From>
+__device__ void store_pairs(const From& pairs, uint16_t* tile, int32_t ld, Stage& stage) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint8_t* region = reinterpret_cast<uint8_t*>(&stage) + wave * 2 * PAIR_BUF;
@@ -597,7 +626,6 @@ __device__ void store_pairs(const v16f acc[4][4], uint16_t* tile, int32_t ld, St
   const __amdgpu_buffer_rsrc_t rsrc =
       __builtin_amdgcn_make_buffer_rsrc(tile, 0, 0x7fffffff, 0x00020000);
   const int32_t lane_off = ((lane >> 3) * ld + 8 * (lane & 7)) * 2;
-  const FromAcc pairs{acc};
   constexpr int M = PH ? 4 : 8;
   auto write = [&](int p) {
     const int i = PH ? p : p >> 1, j0 = PH ? 0 : (p & 1) * 2;
@@ -631,20 +659,61 @@ __device__ void store_pairs(const v16f acc[4][4], uint16_t* tile, int32_t ld, St
 
 // The plain epilogue: the tile's rows [0, rows) and columns [0, cols) of a row-major
 // output of pitch ld, from its corner.
+template <typename T, typename From>
+__device__ __forceinline__ void store_plain(const From& from, T* out, int32_t ld, const Job& j,
+                                            Stage& stage) {
+  if constexpr (std::is_same<T, uint16_t>::value) {
+    if (j.cols >= BN && j.rows >= (j.half ? BM / 2 : BM)) {
+      if (j.half) store_pairs<true>(from, out + j.corner, ld, stage);
+      else store_pairs<false>(from, out + j.corner, ld, stage);
+      return;
+    }
+  }
+  if (j.half) store_tile_half(from, out + j.corner, ld, j.rows, j.cols, stage);
+  else store_tile(from, out + j.corner, ld, j.rows, j.cols, stage);
+}
 template <typename T>
 struct Plain {
   T* out;
   int32_t ld;
   __device__ __forceinline__ void store(const v16f acc[4][4], const Job& j, Stage& stage) const {
-    if constexpr (std::is_same<T, uint16_t>::value) {
-      if (j.cols >= BN && j.rows >= (j.half ? BM / 2 : BM)) {
-        if (j.half) store_pairs<true>(acc, out + j.corner, ld, stage);
-        else store_pairs<false>(acc, out + j.corner, ld, stage);
-        return;
-      }
+    store_plain(FromAcc{acc}, out, ld, j, stage);
+  }
+};
+
+// A lane's biases of its columns, from the group's row at the tile's first column: run g of
+// block b takes columns 8 g + 4 (l / 32) .. + 3 of those 32 (`first` the wave's first).
+template <typename Run, typename T>
+__device__ __forceinline__ void read_bias(Run (&bias)[4][4], const T* row, int32_t first,
+                                          int32_t cols, int32_t blocks) {
+  first += 4 * ((threadIdx.x & 63) >> 5);
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int32_t col = first + b * 32 + 8 * g;  // columns are a multiple of 4
+      bias[b][g] = b < blocks && col < cols ? *reinterpret_cast<const Run*>(row + col) : Run{};
     }
-    if (j.half) store_tile_half(acc, out + j.corner, ld, j.rows, j.cols, stage);
-    else store_tile(acc, out + j.corner, ld, j.rows, j.cols, stage);
+}
+
+// The plain epilogue with each group's row of `bias` (groups, ld) added; the tiles past the
+// groups, which have no K step, stay 0. As a pass of its own the bias of gpt-oss-120b's up
+// GEMM (8192 tokens, 794 us) took 161 us; here the GEMM is 46 us longer, most of it the sums'
+// VALU work, which one wave a SIMD cannot hide (biases through the scalar cache, to keep
+// them from waiting behind the next tile's operands, were no faster).
+template <typename T>
+struct PlainBiased {
+  T* out;
+  int32_t ld;
+  const T* bias;
+  __device__ __forceinline__ void store(const v16f acc[4][4], const Job& j, Stage& stage) const {
+    const int wave = threadIdx.x >> 6;
+    const T* row = bias + static_cast<int64_t>(j.group) * ld + j.b_row0;
+    const int32_t first = j.half ? wave * 64 : (wave & 1) * 128;  // the wave's columns
+    std::conditional_t<std::is_same<T, uint16_t>::value, FromAccBiased16, FromAccBiased32> from{
+        FromAcc{acc}};
+    read_bias(from.bias, row, first, j.n > 0 ? j.cols : 0, j.half ? 2 : 4);
+    store_plain(from, out, ld, j, stage);
   }
 };
 
@@ -701,17 +770,18 @@ struct MxOf {
 using Mx = MxOf<false>;
 
 // The kernels: one workgroup a CU.
-template <typename T, bool W>
+template <typename T, bool W, bool BIASED>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void rows_kernel(
     Operand A, Operand B, int32_t groups, int32_t n, int32_t height,
     const int32_t* __restrict__ starts, const Tile* __restrict__ tiles, int32_t col_tiles,
-    T* __restrict__ y) {
+    const T* __restrict__ bias, T* __restrict__ y) {
   extern __shared__ __align__(16) uint8_t smem[];
   if (!list_fits(starts, groups, A.rows, height)) return;
   Lds& lds = *reinterpret_cast<Lds*>(smem);
   const RowsTiles<false, true> list{tiles, groups, n, height, col_tiles, A.k / BK, A.k};
   const int32_t count = starts[groups + 1] * col_tiles;
-  run_tiles<MxOf<W>>(list, count, A, B, lds, Plain<T>{y, n});
+  if constexpr (BIASED) run_tiles<MxOf<W>>(list, count, A, B, lds, PlainBiased<T>{y, n, bias});
+  else run_tiles<MxOf<W>>(list, count, A, B, lds, Plain<T>{y, n});
 }
 
 // rows_kernel with each group's rows of a from a_starts[g] (the reference's `starts`).
@@ -751,18 +821,23 @@ bool narrow(int64_t rows, int64_t k) { return (rows + BM) * k < (1LL << 31); }
 
 template <typename T, bool W = false>
 int launch_rows(const Operand& A, const Operand& B, int32_t groups, int64_t n, int64_t height,
-                const int32_t* starts, const Tile* tiles, int64_t slots, void* y, hipStream_t s) {
+                const int32_t* starts, const Tile* tiles, int64_t slots, const void* bias, void* y,
+                hipStream_t s) {
   if (!W && !(narrow(A.rows, A.k) && narrow(B.rows, B.k)))
-    return launch_rows<T, true>(A, B, groups, n, height, starts, tiles, slots, y, s);
+    return launch_rows<T, true>(A, B, groups, n, height, starts, tiles, slots, bias, y, s);
   const int64_t col_tiles = ceil_div(n, BN);
   if (slots * col_tiles >= (1LL << 31)) return fail(BUX_E_ARGUMENT, "bux_mx_grouped_rows: too many tiles");
   unsigned blocks = 0;
   if (int rc = grid_for(slots * col_tiles, &blocks)) return rc;
-  if (int rc = allow_lds(rows_kernel<T, W>, sizeof(Lds), "rows_kernel")) return rc;
-  hipLaunchKernelGGL((rows_kernel<T, W>), dim3(blocks), dim3(THREADS), sizeof(Lds), s, A, B, groups,
-                     static_cast<int32_t>(n), static_cast<int32_t>(height), starts, tiles,
-                     static_cast<int32_t>(col_tiles), static_cast<T*>(y));
-  return launched("rows_kernel");
+  auto go = [&](auto kernel) {
+    if (int rc = allow_lds(kernel, sizeof(Lds), "rows_kernel")) return rc;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(THREADS), sizeof(Lds), s, A, B, groups,
+                       static_cast<int32_t>(n), static_cast<int32_t>(height), starts, tiles,
+                       static_cast<int32_t>(col_tiles), static_cast<const T*>(bias),
+                       static_cast<T*>(y));
+    return launched("rows_kernel");
+  };
+  return bias ? go(rows_kernel<T, W, true>) : go(rows_kernel<T, W, false>);
 }
 
 template <typename T, bool W = false>
@@ -1426,7 +1501,8 @@ int check_contract(const char* name, const uint8_t* a_values, const uint8_t* a_s
 
 int launch_rows_of(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b_values,
                    const uint8_t* b_scales, const void* list, int32_t groups, int64_t m, int64_t n,
-                   int64_t k, int64_t height, int out_dtype, void* y, hipStream_t s) {
+                   int64_t k, int64_t height, int out_dtype, void* y, hipStream_t s,
+                   const void* bias = nullptr) {
   // Rows of the groups past a's m rows read 0 (the resource ends there) or the
   // following K chunk's rows: a's m must cover every row the groups hold.
   const Operand A{a_values, a_scales, static_cast<int32_t>(k), static_cast<int32_t>(m)};
@@ -1436,10 +1512,10 @@ int launch_rows_of(const uint8_t* a_values, const uint8_t* a_scales, const uint8
   Tile* tiles = tiles_in(list, groups);
   if (rows_direct(m, groups, n))
     return launch_rows_direct(a_values, a_scales, b_values, b_scales, list, slots, groups, m, n, k,
-                              height, out_dtype, y, s);
+                              height, out_dtype, bias, y, s);
   return out_dtype == BUX_BF16
-             ? launch_rows<uint16_t>(A, B, groups, n, height, starts, tiles, slots, y, s)
-             : launch_rows<float>(A, B, groups, n, height, starts, tiles, slots, y, s);
+             ? launch_rows<uint16_t>(A, B, groups, n, height, starts, tiles, slots, bias, y, s)
+             : launch_rows<float>(A, B, groups, n, height, starts, tiles, slots, bias, y, s);
 }
 
 int launch_contract_of(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b_values,
@@ -1628,6 +1704,27 @@ extern "C" int bux_mx_grouped_rows_listed(const uint8_t* a_values, const uint8_t
   if (height == 0) return BUX_OK;
   return launch_rows_of(a_values, a_scales, b_values, b_scales, list, groups, m, n, k, height,
                         out_dtype, y, as_stream(stream));
+}
+
+extern "C" int bux_mx_grouped_rows_biased(const uint8_t* a_values, const uint8_t* a_scales,
+                                          const uint8_t* b_values, const uint8_t* b_scales,
+                                          void* list, size_t list_bytes, int32_t groups,
+                                          int64_t m, int64_t n, int64_t k, int64_t height,
+                                          int out_dtype, const void* bias, void* y, void* stream) {
+  using namespace bux;
+  const char* const name = "bux_mx_grouped_rows_biased";
+  clear_error();
+  if (int rc = check_rows(name, a_values, a_scales, b_values, b_scales, groups, m, n, k, height,
+                          out_dtype, y))
+    return rc;
+  BUX_CHECK(list != nullptr && bias != nullptr, "%s: NULL list or bias", name);
+  const size_t need = bux_mx_grouped_rows_workspace_size(groups, m, height);
+  if (list_bytes < need)
+    return fail(BUX_E_WORKSPACE, "%s: a list of %zu bytes, not one for groups=%d m=%lld height=%lld "
+                "(%zu bytes)", name, list_bytes, groups, (long long)m, (long long)height, need);
+  if (height == 0) return BUX_OK;
+  return launch_rows_of(a_values, a_scales, b_values, b_scales, list, groups, m, n, k, height,
+                        out_dtype, y, as_stream(stream), bias);
 }
 
 extern "C" size_t bux_mx_grouped_contract_workspace_size(int32_t groups) {

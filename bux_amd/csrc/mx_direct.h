@@ -11,10 +11,11 @@ namespace bux {
 bool rows_direct(int64_t m, int32_t groups, int64_t n);
 
 // As grouped_mx.hip's launch_rows: `list` a tile list of `slots` records (its starts
-// before them), the operands in the tiled layout, y (height, n) of out_dtype.
+// before them), the operands in the tiled layout, `bias` NULL or
+// (groups, n) of out_dtype, y (height, n) of it.
 int launch_rows_direct(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b_values,
                        const uint8_t* b_scales, const void* list, int64_t slots, int32_t groups,
-                       int64_t m, int64_t n, int64_t k, int64_t height, int out_dtype, void* y,
-                       hipStream_t s);
+                       int64_t m, int64_t n, int64_t k, int64_t height, int out_dtype,
+                       const void* bias, void* y, hipStream_t s);
 
 }  // namespace bux

@@ -57,7 +57,8 @@ __global__ __launch_bounds__(64) void rows_direct_kernel(
     const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_scales,
     const uint8_t* __restrict__ b_values, const uint8_t* __restrict__ b_scales, int32_t k,
     int32_t a_rows, int32_t n, int32_t groups, int32_t height, const int32_t* __restrict__ starts,
-    const Tile* __restrict__ tiles, int32_t col_blocks, T* __restrict__ y) {
+    const Tile* __restrict__ tiles, int32_t col_blocks, const T* __restrict__ bias,
+    T* __restrict__ y) {
   if (!list_fits(starts, groups, a_rows, height)) return;
   const int32_t id = blockIdx.x / col_blocks;
   if (id >= starts[groups + 1]) return;
@@ -155,7 +156,12 @@ __global__ __launch_bounds__(64) void rows_direct_kernel(
       const int32_t col = col0 + 32 * j + 8 * g + 4 * half;
       if (col >= n) continue;  // n is a multiple of 4
       T* at = y + static_cast<int64_t>(row) * n + col;
-      const float c[4] = {acc[j][4 * g], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]};
+      float c[4] = {acc[j][4 * g], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]};
+      if (bias != nullptr && pairs > 0) {  // the product rounded, then the sum
+        const T* b = bias + static_cast<int64_t>(group) * n + col;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) c[q] = Elem<T>::round(c[q]) + Elem<T>::value(b[q]);
+      }
       if constexpr (std::is_same<T, uint16_t>::value)
         *reinterpret_cast<uint2*>(at) = make_uint2(pack_bf16x2(c[0], c[1]), pack_bf16x2(c[2], c[3]));
       else
@@ -166,7 +172,7 @@ __global__ __launch_bounds__(64) void rows_direct_kernel(
 template <typename T>
 int launch_as(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b_values,
               const uint8_t* b_scales, const void* list, int64_t slots, int32_t groups, int64_t m,
-              int64_t n, int64_t k, int64_t height, void* y, hipStream_t s) {
+              int64_t n, int64_t k, int64_t height, const void* bias, void* y, hipStream_t s) {
   const int64_t col_blocks = ceil_div(n, 32 * CB);
   if (slots * col_blocks >= (1LL << 31)) return fail(BUX_E_ARGUMENT, "bux_mx_grouped_rows: too many tiles");
   const int64_t rows = m > height ? m : height;  // no tile holds more
@@ -176,7 +182,7 @@ int launch_as(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b
                      dim3(64), 0, s, a_values, a_scales, b_values, b_scales, static_cast<int32_t>(k),
                      static_cast<int32_t>(m), static_cast<int32_t>(n), groups,
                      static_cast<int32_t>(height), starts_in(list), tiles_in(list, groups),
-                     static_cast<int32_t>(col_blocks), static_cast<T*>(y));
+                     static_cast<int32_t>(col_blocks), static_cast<const T*>(bias), static_cast<T*>(y));
   return launched("rows_direct_kernel");
 }
 
@@ -196,13 +202,13 @@ bool rows_direct(int64_t m, int32_t groups, int64_t n) {
 
 int launch_rows_direct(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b_values,
                        const uint8_t* b_scales, const void* list, int64_t slots, int32_t groups,
-                       int64_t m, int64_t n, int64_t k, int64_t height, int out_dtype, void* y,
-                       hipStream_t s) {
+                       int64_t m, int64_t n, int64_t k, int64_t height, int out_dtype,
+                       const void* bias, void* y, hipStream_t s) {
   return out_dtype == BUX_BF16
              ? launch_as<uint16_t>(a_values, a_scales, b_values, b_scales, list, slots, groups, m, n,
-                                   k, height, y, s)
+                                   k, height, bias, y, s)
              : launch_as<float>(a_values, a_scales, b_values, b_scales, list, slots, groups, m, n, k,
-                                height, y, s);
+                                height, bias, y, s);
 }
 
 }  // namespace bux

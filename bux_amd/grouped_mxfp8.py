@@ -197,6 +197,7 @@ def tiles_of(sizes: torch.Tensor, m: int, height: int) -> TileList:
 def rows(
     a: Tiled, b: Tiled, sizes: torch.Tensor, out: torch.dtype = torch.bfloat16,
     height: int | None = None, tiles: TileList | None = None, starts: torch.Tensor | None = None,
+    bias: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """Return ``a @ b[g]^T`` for each group g's rows of a, (height, n), the rows past
     the groups 0.
@@ -212,6 +213,8 @@ def rows(
         starts: int32 (g,) on the device: where each group's rows of a start (the
             reference's `starts`, grouped_mxfp8.py:116-154); None for packed. y's rows
             stay packed either way.
+        bias: with `tiles`, each group's row of (g, n), in `out`'s dtype, added to its
+            rows' rounded products (``moe.add_expert_bias`` of the result).
     """
     require(a.values, a.scales, b.values, b.scales, sizes)
     if a.values.dim() != 3 or b.values.dim() != 4:
@@ -223,6 +226,11 @@ def rows(
         raise ValueError(f"rows: a {tuple(a.values.shape)}, b {tuple(b.values.shape)}, "
                          f"sizes {tuple(sizes.shape)} {sizes.dtype}")
     h = m if height is None else height
+    if bias is not None:
+        require(bias)
+        if tiles is None or bias.dtype != out or bias.numel() != groups * n:
+            raise ValueError(f"rows: bias {bias.dtype} {tuple(bias.shape)} for {groups} groups of {n} "
+                             f"columns in {out}, with a tile list")
     y = torch.empty(h, n, dtype=out, device=a.values.device)
     if starts is not None:
         require(starts)
@@ -238,6 +246,11 @@ def rows(
         if (tiles.groups, tiles.m, tiles.height) != (groups, m, h):
             raise ValueError(f"rows: a tile list for {tiles.groups} groups, m={tiles.m}, "
                              f"height={tiles.height}, not {groups}, {m}, {h}")
+        if bias is not None:
+            _lib.check(lib().bux_mx_grouped_rows_biased(
+                ptr(a.values), ptr(a.scales), ptr(b.values), ptr(b.scales), ptr(tiles.buffer),
+                tiles.buffer.numel(), groups, m, n, k, h, _DTYPES[out], ptr(bias), ptr(y), stream()))
+            return y
         _lib.check(lib().bux_mx_grouped_rows_listed(
             ptr(a.values), ptr(a.scales), ptr(b.values), ptr(b.scales), ptr(tiles.buffer),
             tiles.buffer.numel(), groups, m, n, k, h, _DTYPES[out], ptr(y), stream()))

@@ -636,11 +636,13 @@ def experts_forward(
                                                           ffn.struct(True), m)
     else:
         with span("up fprop"):
-            if fprop:
-                projected = grouped_mxfp8.rows(x_k, up_k, s.sizes, dt, height=m, tiles=listed)
+            if fprop:  # the bias in the GEMM's epilogue
+                projected = grouped_mxfp8.rows(
+                    x_k, up_k, s.sizes, dt, height=m, tiles=listed,
+                    bias=None if up_bias is None else up_bias.reshape(e, f * p).contiguous())
             else:
                 projected = grouped.dot(rows, up2, s.sizes)
-        if up_bias is not None:
+        if up_bias is not None and not fprop:
             with span("up bias"):
                 add_expert_bias(projected, up_bias.reshape(e, f * p), s.offsets)
         pv = projected.view(m, f, p)

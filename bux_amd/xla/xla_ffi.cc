@@ -193,6 +193,18 @@ XLA_FFI_DEFINE_HANDLER_SYMBOL(BuxMxRowsListed, MxRowsListed,
                               ffi::Ffi::Bind().Ctx<Stream>().Arg<In>().Arg<In>().Arg<In>()
                                   .Arg<In>().Arg<In>().Ret<In>());
 
+// bias [groups, n] in y's dtype.
+static ffi::Error MxRowsBiased(hipStream_t s, In av, In as, In bv, In bs, In list, In bias,
+                               Out y) {
+  return status(bux_mx_grouped_rows_biased(
+      at<const uint8_t>(av), at<const uint8_t>(as), at<const uint8_t>(bv), at<const uint8_t>(bs),
+      at<void>(list), list.size_bytes(), static_cast<int32_t>(dim(bv, 0)), dim(av, 1), dim(bv, 2),
+      dim(av, 0) * 64, dim(y, 0), dtype_of(y), at<const void>(bias), at<void>(y), s));
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(BuxMxRowsBiased, MxRowsBiased,
+                              ffi::Ffi::Bind().Ctx<Stream>().Arg<In>().Arg<In>().Arg<In>()
+                                  .Arg<In>().Arg<In>().Arg<In>().Ret<In>());
+
 static ffi::Error MxContract(hipStream_t s, In av, In as, In bv, In bs, In sizes, Out dw,
                              Out ws) {
   return status(bux_mx_grouped_contract(

@@ -205,6 +205,15 @@ int bux_mx_grouped_rows_listed(const uint8_t* a_values, const uint8_t* a_scales,
                                const uint8_t* b_values, const uint8_t* b_scales, void* list,
                                size_t list_bytes, int32_t groups, int64_t m, int64_t n, int64_t k,
                                int64_t height, int out_dtype, void* y, void* stream);
+/* bux_mx_grouped_rows_biased: bux_mx_grouped_rows_listed with each group's row of `bias`
+ * [groups, n] (of out_dtype) added to its rows as an op of its own adds it (the product
+ * rounded to out_dtype, then the sum: bux_expert_bias_add's result to the bit; the
+ * reference's up bias, experts/moe.py:857-861). The rows past the groups stay 0. */
+int bux_mx_grouped_rows_biased(const uint8_t* a_values, const uint8_t* a_scales,
+                               const uint8_t* b_values, const uint8_t* b_scales, void* list,
+                               size_t list_bytes, int32_t groups, int64_t m, int64_t n, int64_t k,
+                               int64_t height, int out_dtype, const void* bias, void* y,
+                               void* stream);
 int bux_mx_grouped_contract_listed(const uint8_t* a_values, const uint8_t* a_scales,
                                    const uint8_t* b_values, const uint8_t* b_scales, void* list,
                                    size_t list_bytes, int32_t groups, int64_t d, int64_t f,

@@ -1,0 +1,71 @@
+"""The rows GEMM's bias epilogue against the bias added as an op of its own, to the bit, over
+whole, half and partial tiles, empty groups, rows past the groups and the kernel for groups
+of few rows; and the biased token sums, whose experts are found a token at once, against
+float64 at every k around its kernels' 4 and 8 picks."""
+
+import numpy as np
+import pytest
+import torch
+
+from tests._util import announce
+from tests.test_gpu_small_groups import _codes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("sizes,k,n", [([300, 0, 129, 256], 256, 512), ([700, 90], 128, 516),
+                                       ([256, 100, 511], 384, 36), ([3, 0, 40] + [1] * 60, 256, 132)])
+def test_rows_with_a_bias(lib, sizes, k, n, dtype):
+    from bux_amd import grouped_mxfp8, moe
+    rng = np.random.default_rng(100)
+    filled = sum(sizes)
+    m = filled + 30
+    gs = torch.tensor(sizes, dtype=torch.int32, device="cuda")
+    offsets = torch.tensor([0, *np.cumsum(sizes)], dtype=torch.int32, device="cuda")
+    a, b = _codes(rng, (m, k)), _codes(rng, (len(sizes), n, k))
+    bias = (torch.randn(len(sizes), n, device="cuda") * 100).to(dtype)
+    tiles = grouped_mxfp8.tiles_of(gs, m, m)
+    announce("rows with a bias", sizes[:4], k, n, dtype)
+    got = grouped_mxfp8.rows(a, b, gs, dtype, tiles=tiles, bias=bias)
+    plain = grouped_mxfp8.rows(a, b, gs, dtype, tiles=tiles)
+    expert = torch.repeat_interleave(torch.arange(len(sizes), device="cuda"), gs.long())
+    want = plain.clone()
+    want[:filled] += bias[expert]
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and not torch.equal(got, plain)
+    assert (got[filled:] == 0).all()
+    if n % 8 == 0:
+        assert torch.equal(got, moe.add_expert_bias(plain, bias, offsets))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("k,experts,width", [(1, 1, 8), (3, 64, 264), (4, 65, 2880), (5, 200, 2056),
+                                             (8, 128, 1024), (9, 70, 264)])
+def test_biased_token_sums(lib, k, experts, width, dtype):
+    from bux_amd import moe
+    g = torch.Generator(device="cuda").manual_seed(101)
+    t = 37
+    idx = torch.randint(-1, experts + 1, (t, k), generator=g, device="cuda").int()  # some in no expert
+    s = moe.sort_by_expert(idx, experts)
+    y, bias = (torch.randn(*shape, generator=g, device="cuda").to(dtype)
+               for shape in ((t * k, width), (experts, width)))
+    w = torch.randn(t * k, generator=g, device="cuda").to(dtype)
+    inverse = s.inverse.view(t, k).clone()
+    inverse[0, 0] = t * k  # a row outside y adds nothing
+    announce("biased token sums", k, experts, width, dtype)
+    got = moe.sum_by_token_biased(y, inverse, bias, s.offsets, w)
+    torch.cuda.synchronize()
+    expert = idx.long().clamp(0, experts - 1)
+    inside = (idx >= 0) & (idx < experts)
+    inside[0, 0] = False
+    rows = inverse.long().clamp(max=t * k - 1)
+    part = (bias[expert] * w[rows][..., None]).double() * inside[..., None]
+    there = torch.ones(t, k, 1, device="cuda", dtype=torch.float64)
+    there[0, 0] = 0
+    both = [(y[rows].double() * there).sum(1), part.sum(1)]
+    # each float32 sum of k terms, then (bfloat16) its rounding and the total's
+    unit = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-23
+    size = (y[rows].double() * there).abs().sum(1) + part.abs().sum(1)
+    bound = k * 2.0**-24 * size + unit * (both[0].abs() + both[1].abs()) + unit * sum(both).abs()
+    assert bool(((got.double() - sum(both)).abs() <= bound).all())
