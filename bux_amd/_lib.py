@@ -160,6 +160,11 @@ class BuxError(RuntimeError):
 _LIB = None
 
 
+def built() -> bool:
+    """Return whether the library is there: loaded, or its file."""
+    return _LIB is not None or os.path.exists(PATH)
+
+
 def load(path: str = PATH) -> ctypes.CDLL:
     """Return the library, loaded once, each entry point typed. Raises if it is not
     built."""

@@ -41,17 +41,27 @@ class Spans:
         return out
 
 
-@contextlib.contextmanager
+class _Span:
+    """One timed block of an active `Spans`."""
+
+    def __init__(self, spans: Spans, name: str) -> None:
+        self.spans, self.name = spans, name
+
+    def __enter__(self) -> None:
+        self.start = torch.cuda.Event(enable_timing=True)
+        self.start.record()
+
+    def __exit__(self, kind, *exc) -> None:
+        if kind is None:
+            end = torch.cuda.Event(enable_timing=True)
+            end.record()
+            self.spans.events[self.name].append((self.start, end))
+
+
+_UNTIMED = contextlib.nullcontext()
+
+
 def span(name: str):
     """Time what the block enqueues on the current stream under `name`, if a `Spans` is
     active."""
-    spans = _ACTIVE
-    if spans is None:
-        yield
-        return
-    start = torch.cuda.Event(enable_timing=True)
-    end = torch.cuda.Event(enable_timing=True)
-    start.record()
-    yield
-    end.record()
-    spans.events[name].append((start, end))
+    return _UNTIMED if _ACTIVE is None else _Span(_ACTIVE, name)
