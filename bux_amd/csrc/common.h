@@ -91,6 +91,40 @@ __device__ __forceinline__ float power_of_two_down(int e) {
 
 __device__ __forceinline__ float clip448(float v) { return fminf(fmaxf(v, -448.0f), 448.0f); }
 
+// --- blocks of bfloat16 -------------------------------------------------------------
+
+// The quantizers of bfloat16 blocks work on packed pairs: a block's largest magnitude as
+// an integer maximum of the pairs' bits, its codes by gfx950's v_cvt_scalef32_pk_fp8_bf16,
+// two bfloat16 over a power of two to two E4M3 at once. For a finite block whose values
+// over 2^e lie within +-448 these are the bits of the float route (widen, multiply by
+// 2^-e, clip, convert): checked on the MI355X for every finite bfloat16 and every e. A
+// block that holds an infinity or a NaN (`top` past FINITE_BF16) takes the float route,
+// whose maximum passes NaN over and whose clip bounds infinities.
+constexpr uint32_t FINITE_BF16 = 0x7f7f;
+
+// The larger of each half, ignoring signs.
+__device__ __forceinline__ uint32_t max_abs_pair(uint32_t m, uint32_t pair) {
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, m),
+                                                                __builtin_bit_cast(u16x2, pair & 0x7fff7fffu)));
+}
+__device__ __forceinline__ uint32_t larger_half(uint32_t m) {
+  return (m & 0xffffu) > (m >> 16) ? (m & 0xffffu) : (m >> 16);
+}
+// Four bfloat16 (two pairs) over `scale`, a power of two, to four codes.
+__device__ __forceinline__ uint32_t e4m3x4_bf16(uint32_t lo, uint32_t hi, float scale) {
+  typedef short s16x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  s16x2 r = {0, 0};
+  r = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(r, __builtin_bit_cast(bf16x2, lo), scale, false);
+  r = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(r, __builtin_bit_cast(bf16x2, hi), scale, true);
+  return __builtin_bit_cast(uint32_t, r);
+}
+// 2^e as a float32, exactly, for e in [-126, 126].
+__device__ __forceinline__ float power_of_two(int e) {
+  return __uint_as_float(static_cast<uint32_t>(127 + e) << 23);
+}
+
 // --- the layer's element types ----------------------------------------------------
 
 // A layer computes in its tokens' dtype (the reference's x.dtype, experts/moe.py:846):

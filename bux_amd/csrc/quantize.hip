@@ -34,6 +34,10 @@
 //     tile's 128 rows as one word. The tile's 16-byte chunks are swizzled by row (chunk
 //     c of row r at c ^ 2 ((r / 16) % 4)), so that the four lanes' rows, 16 apart, read
 //     different banks.
+// bfloat16 blocks are reduced and converted as packed pairs (common.h's e4m3x4_bf16): the
+// quantizers by index and of the activations' gradients issued too many VALU instructions to
+// keep up with memory (config 3: the tokens by index 171 -> 153 us, h 126 -> 121, d projected
+// 233 -> 215, W_up 283 -> 280; DeepSeek-V3's tokens 300 -> 291).
 // HBM traffic per element: 2 bytes read (4 of float32), 2 x (1 + 1/32) bytes written; the
 // codes go out as non-temporal stores (below).
 //
@@ -413,20 +417,42 @@ __global__ __launch_bounds__(THREADS) void quantize_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int64_t r = row0 + (t >> 3) + 32 * i;
-      float v[8];
-      P8::floats(raw[i], v);
-      float amax = 0.0f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-      amax = fmaxf(amax, __shfl_xor(amax, 1));
-      amax = fmaxf(amax, __shfl_xor(amax, 2));
-      const int e = tiles ? tile_e(i, chunk >> 2) : P8::exponent(amax);
-      const float down = power_of_two_down(e);
       uint2 codes;
-      codes.x = e4m3x4(clip448(v[0] * down), clip448(v[1] * down), clip448(v[2] * down),
-                       clip448(v[3] * down));
-      codes.y = e4m3x4(clip448(v[4] * down), clip448(v[5] * down), clip448(v[6] * down),
-                       clip448(v[7] * down));
+      int e;
+      // a row's block of 32 is 4 neighbouring lanes
+      auto by_floats = [&] {
+        float v[8];
+        P8::floats(raw[i], v);
+        float amax = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
+        amax = fmaxf(amax, __shfl_xor(amax, 1));
+        amax = fmaxf(amax, __shfl_xor(amax, 2));
+        e = tiles ? tile_e(i, chunk >> 2) : P8::exponent(amax);
+        const float down = power_of_two_down(e);
+        codes.x = e4m3x4(clip448(v[0] * down), clip448(v[1] * down), clip448(v[2] * down),
+                         clip448(v[3] * down));
+        codes.y = e4m3x4(clip448(v[4] * down), clip448(v[5] * down), clip448(v[6] * down),
+                         clip448(v[7] * down));
+      };
+      if constexpr (std::is_same<V, uint16_t>::value) {
+        uint32_t m = max_abs_pair(raw[i].x & 0x7fff7fffu, raw[i].y);
+        m = max_abs_pair(max_abs_pair(m, raw[i].z), raw[i].w);
+        uint32_t top = larger_half(m), other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), 1));
+        top = top > other ? top : other;
+        other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), 2));
+        top = top > other ? top : other;
+        if (top <= FINITE_BF16) {  // the same in the block's lanes
+          e = tiles ? tile_e(i, chunk >> 2) : P8::exponent(__uint_as_float(top << 16));
+          const float scale = power_of_two(e);
+          codes.x = e4m3x4_bf16(raw[i].x, raw[i].y, scale);
+          codes.y = e4m3x4_bf16(raw[i].z, raw[i].w, scale);
+        } else {
+          by_floats();
+        }
+      } else {
+        by_floats();
+      }
       if (r < height) {  // padding columns too: codes 0, scale byte 1
         stream_codes(vg + ((col >> 6) * height + r) * 64 + (col & 63), codes.x, codes.y);
         const int64_t b = col >> 5;
@@ -453,21 +479,49 @@ __global__ __launch_bounds__(THREADS) void quantize_kernel(
   uint32_t word = 0;  // lane 0's scale bytes of the 4 blocks
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    float v[16];
-    float amax = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      v[j] = P8::widen(at(64 * h + 16 * q + j, lc));
-      amax = fmaxf(amax, fabsf(v[j]));
-    }
-    amax = fmaxf(amax, __shfl_xor(amax, 1));
-    const int e = tiles ? tile_e(2 * h + (q >> 1), lc >> 5) : P8::exponent(amax);
-    const float down = power_of_two_down(e);
     uint32_t w[4];
+    int e;
+    V x[16];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      w[j] = e4m3x4(clip448(v[4 * j] * down), clip448(v[4 * j + 1] * down),
-                    clip448(v[4 * j + 2] * down), clip448(v[4 * j + 3] * down));
+    for (int j = 0; j < 16; ++j) x[j] = at(64 * h + 16 * q + j, lc);
+    // a column's block of 32 is 2 neighbouring lanes
+    auto by_floats = [&] {
+      float v[16];
+      float amax = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        v[j] = P8::widen(x[j]);
+        amax = fmaxf(amax, fabsf(v[j]));
+      }
+      amax = fmaxf(amax, __shfl_xor(amax, 1));
+      e = tiles ? tile_e(2 * h + (q >> 1), lc >> 5) : P8::exponent(amax);
+      const float down = power_of_two_down(e);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        w[j] = e4m3x4(clip448(v[4 * j] * down), clip448(v[4 * j + 1] * down),
+                      clip448(v[4 * j + 2] * down), clip448(v[4 * j + 3] * down));
+    };
+    if constexpr (std::is_same<V, uint16_t>::value) {
+      uint32_t pair[8], m = 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        pair[j] = static_cast<uint32_t>(x[2 * j]) | (static_cast<uint32_t>(x[2 * j + 1]) << 16);
+        m = max_abs_pair(m, pair[j]);
+      }
+      uint32_t top = larger_half(m);
+      const uint32_t other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), 1));
+      top = top > other ? top : other;
+      if (top <= FINITE_BF16) {
+        e = tiles ? tile_e(2 * h + (q >> 1), lc >> 5) : P8::exponent(__uint_as_float(top << 16));
+        const float scale = power_of_two(e);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = e4m3x4_bf16(pair[2 * j], pair[2 * j + 1], scale);
+      } else {
+        by_floats();
+      }
+    } else {
+      by_floats();
+    }
     if (col_out) stream_codes(out + h * cols * 64, w[0], w[1], w[2], w[3]);
     // block 2 h from this pair (q 0, 1), block 2 h + 1 from the other (q 2, 3)
     const uint32_t b = static_cast<uint32_t>(e + 127);
