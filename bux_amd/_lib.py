@@ -90,6 +90,12 @@ SIGNATURES = {
     "bux_bf16_grouped_rows_f32": (
         _int, [_p, _p, _int, _p, _i32, _i64, _i64, _i64, _p, _p, _size, _p]),
     "bux_bf16_grouped_contract_f32": (_int, [_p, _p, _p, _i32, _i64, _i64, _i64, _p, _p, _size, _p]),
+    "bux_bf16_grouped_rows_listed": (_int, [_p, _p, _int, _i32, _i64, _i64, _i64, _p, _p, _size, _p]),
+    "bux_bf16_grouped_rows_listed_f32": (
+        _int, [_p, _p, _int, _i32, _i64, _i64, _i64, _p, _p, _size, _p]),
+    "bux_bf16_grouped_contract_listed": (_int, [_p, _p, _i32, _i64, _i64, _i64, _p, _p, _size, _p]),
+    "bux_bf16_grouped_contract_listed_f32": (
+        _int, [_p, _p, _i32, _i64, _i64, _i64, _p, _p, _size, _p]),
     "bux_token_rows": (_int, [_p, _i64, _p, _i64, _i32, _i64, _p, _p]),
     "bux_token_sums": (_int, [_p, _i64, _p, _i64, _i32, _i64, _p, _p]),
     "bux_token_sums_f32": (_int, [_p, _i64, _p, _i64, _i32, _i64, _p, _p]),

@@ -767,28 +767,30 @@ extern "C" size_t bux_bf16_grouped_rows_workspace_size(int32_t groups, int64_t m
   return starts_bytes(groups) + static_cast<size_t>(row_slots(groups, m, m)) * sizeof(Tile);
 }
 
-extern "C" int bux_bf16_grouped_rows(const uint16_t* x, const uint16_t* w, int w_transposed,
+// With `sizes` NULL, the workspace is a list already made of them (the _listed entry points).
+static int rows_on(const uint16_t* x, const uint16_t* w, int w_transposed,
                                      const int32_t* sizes, int32_t groups, int64_t m, int64_t n,
                                      int64_t k, uint16_t* y, void* workspace,
                                      size_t workspace_bytes, void* stream) {
   using namespace bux;
-  clear_error();
   BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS, "bux_bf16_grouped_rows: groups=%d outside [1, %d]",
             groups, MAX_GROUPS);
   BUX_CHECK(m >= 0 && n > 0 && k > 0, "bux_bf16_grouped_rows: bad shape m=%lld n=%lld k=%lld",
             (long long)m, (long long)n, (long long)k);
   BUX_CHECK(m < INT32_MAX, "bux_bf16_grouped_rows: m=%lld rows", (long long)m);
-  BUX_CHECK(sizes && w && y && (m == 0 || x), "bux_bf16_grouped_rows: NULL buffer");
+  BUX_CHECK(w && y && (m == 0 || x), "bux_bf16_grouped_rows: NULL buffer");
   const size_t need = bux_bf16_grouped_rows_workspace_size(groups, m);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(BUX_E_WORKSPACE, "bux_bf16_grouped_rows: workspace of %zu bytes, %zu needed",
                 workspace_bytes, need);
   if (m == 0) return BUX_OK;
   hipStream_t s = as_stream(stream);
-  hipLaunchKernelGGL(prologue_kernel, dim3(1), dim3(THREADS), 0, s, sizes, groups, m,
-                     row_slots(groups, m, m), 1, starts_in(workspace), tiles_in(workspace, groups),
-                     header_in(workspace), m, nullptr);
-  if (int rc = launched("prologue_kernel")) return rc;
+  if (sizes) {
+    hipLaunchKernelGGL(prologue_kernel, dim3(1), dim3(THREADS), 0, s, sizes, groups, m,
+                       row_slots(groups, m, m), 1, starts_in(workspace), tiles_in(workspace, groups),
+                       header_in(workspace), m, nullptr);
+    if (int rc = launched("prologue_kernel")) return rc;
+  }
   // n or k off 16-byte rows, or an operand past 32-bit offsets: the any-shape kernel
   if (n % 8 != 0 || k % 8 != 0 || !fits(m, k) || !(w_transposed ? fits(n, k) : fits(k, n))) {
     const int64_t col_tiles = ceil_div(n, ANY_BN), slots = row_slots(groups, m, m);
@@ -814,32 +816,51 @@ extern "C" int bux_bf16_grouped_rows(const uint16_t* x, const uint16_t* w, int w
               : launch_rows<false, false>(A, B, groups, m, n, k, workspace, s, y);
 }
 
+extern "C" int bux_bf16_grouped_rows(const uint16_t* x, const uint16_t* w, int w_transposed,
+                                     const int32_t* sizes, int32_t groups, int64_t m, int64_t n,
+                                     int64_t k, uint16_t* y, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
+  using namespace bux;
+  clear_error();
+  BUX_CHECK(sizes != nullptr, "bux_bf16_grouped_rows: NULL buffer");
+  return rows_on(x, w, w_transposed, sizes, groups, m, n, k, y, workspace, workspace_bytes, stream);
+}
+
+extern "C" int bux_bf16_grouped_rows_listed(const uint16_t* x, const uint16_t* w, int w_transposed,
+                                     int32_t groups, int64_t m, int64_t n,
+                                     int64_t k, uint16_t* y, void* list,
+                                     size_t list_bytes, void* stream) {
+  bux::clear_error();
+  return rows_on(x, w, w_transposed, nullptr, groups, m, n, k, y, list, list_bytes, stream);
+}
+
 extern "C" size_t bux_bf16_grouped_contract_workspace_size(int32_t groups) {
   using namespace bux;
   return starts_bytes(groups);  // the group starts alone: header, starts
 }
 
-extern "C" int bux_bf16_grouped_contract(const uint16_t* x, const uint16_t* dy, const int32_t* sizes,
+static int contract_on(const uint16_t* x, const uint16_t* dy, const int32_t* sizes,
                                          int32_t groups, int64_t m, int64_t k, int64_t n,
                                          uint16_t* dw, void* workspace, size_t workspace_bytes,
                                          void* stream) {
   using namespace bux;
-  clear_error();
   BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS,
             "bux_bf16_grouped_contract: groups=%d outside [1, %d]", groups, MAX_GROUPS);
   BUX_CHECK(m >= 0 && n > 0 && k > 0, "bux_bf16_grouped_contract: bad shape m=%lld k=%lld n=%lld",
             (long long)m, (long long)k, (long long)n);
   BUX_CHECK(m < INT32_MAX, "bux_bf16_grouped_contract: m=%lld rows", (long long)m);
-  BUX_CHECK(sizes && dw && (m == 0 || (x && dy)), "bux_bf16_grouped_contract: NULL buffer");
+  BUX_CHECK(dw && (m == 0 || (x && dy)), "bux_bf16_grouped_contract: NULL buffer");
   const size_t need = bux_bf16_grouped_contract_workspace_size(groups);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(BUX_E_WORKSPACE, "bux_bf16_grouped_contract: workspace of %zu bytes, %zu needed",
                 workspace_bytes, need);
   hipStream_t s = as_stream(stream);
   // the starts capped at the contract's K (m rows), as the rows GEMM caps them at its rows
-  hipLaunchKernelGGL(prologue_kernel, dim3(1), dim3(THREADS), 0, s, sizes, groups, 0, 0, 1,
-                     starts_in(workspace), nullptr, header_in(workspace), m, nullptr);
-  if (int rc = launched("prologue_kernel")) return rc;
+  if (sizes) {
+    hipLaunchKernelGGL(prologue_kernel, dim3(1), dim3(THREADS), 0, s, sizes, groups, 0, 0, 1,
+                       starts_in(workspace), nullptr, header_in(workspace), m, nullptr);
+    if (int rc = launched("prologue_kernel")) return rc;
+  }
   if (n % 8 != 0 || k % 8 != 0 || !fits(m, k) || !fits(m, n)) {  // the any-shape kernel
     const int64_t k_tiles = ceil_div(k, BM), col_tiles = ceil_div(n, ANY_BN);
     const int64_t blocks = static_cast<int64_t>(groups) * k_tiles * col_tiles;
@@ -863,28 +884,46 @@ extern "C" int bux_bf16_grouped_contract(const uint16_t* x, const uint16_t* dy, 
   return launched("bf16 contract_kernel");
 }
 
-extern "C" int bux_bf16_grouped_rows_f32(const float* x, const float* w, int w_transposed,
+extern "C" int bux_bf16_grouped_contract(const uint16_t* x, const uint16_t* dy, const int32_t* sizes,
+                                         int32_t groups, int64_t m, int64_t k, int64_t n,
+                                         uint16_t* dw, void* workspace, size_t workspace_bytes,
+                                         void* stream) {
+  using namespace bux;
+  clear_error();
+  BUX_CHECK(sizes != nullptr, "bux_bf16_grouped_contract: NULL buffer");
+  return contract_on(x, dy, sizes, groups, m, k, n, dw, workspace, workspace_bytes, stream);
+}
+
+extern "C" int bux_bf16_grouped_contract_listed(const uint16_t* x, const uint16_t* dy, int32_t groups, int64_t m, int64_t k, int64_t n,
+                                         uint16_t* dw, void* list, size_t list_bytes,
+                                         void* stream) {
+  bux::clear_error();
+  return contract_on(x, dy, nullptr, groups, m, k, n, dw, list, list_bytes, stream);
+}
+
+static int rows_f32_on(const float* x, const float* w, int w_transposed,
                                          const int32_t* sizes, int32_t groups, int64_t m,
                                          int64_t n, int64_t k, float* y, void* workspace,
                                          size_t workspace_bytes, void* stream) {
   using namespace bux;
-  clear_error();
   BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS,
             "bux_bf16_grouped_rows_f32: groups=%d outside [1, %d]", groups, MAX_GROUPS);
   BUX_CHECK(m >= 0 && n > 0 && k > 0, "bux_bf16_grouped_rows_f32: bad shape m=%lld n=%lld k=%lld",
             (long long)m, (long long)n, (long long)k);
   BUX_CHECK(m < INT32_MAX, "bux_bf16_grouped_rows_f32: m=%lld rows", (long long)m);
-  BUX_CHECK(sizes && w && y && (m == 0 || x), "bux_bf16_grouped_rows_f32: NULL buffer");
+  BUX_CHECK(w && y && (m == 0 || x), "bux_bf16_grouped_rows_f32: NULL buffer");
   const size_t need = bux_bf16_grouped_rows_workspace_size(groups, m);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(BUX_E_WORKSPACE, "bux_bf16_grouped_rows_f32: workspace of %zu bytes, %zu needed",
                 workspace_bytes, need);
   if (m == 0) return BUX_OK;
   hipStream_t s = as_stream(stream);
-  hipLaunchKernelGGL(prologue_kernel, dim3(1), dim3(THREADS), 0, s, sizes, groups, m,
-                     row_slots(groups, m, m), 1, starts_in(workspace), tiles_in(workspace, groups),
-                     header_in(workspace), m, nullptr);
-  if (int rc = launched("prologue_kernel")) return rc;
+  if (sizes) {
+    hipLaunchKernelGGL(prologue_kernel, dim3(1), dim3(THREADS), 0, s, sizes, groups, m,
+                       row_slots(groups, m, m), 1, starts_in(workspace), tiles_in(workspace, groups),
+                       header_in(workspace), m, nullptr);
+    if (int rc = launched("prologue_kernel")) return rc;
+  }
   const int64_t col_tiles = ceil_div(n, ANY_BN), slots = row_slots(groups, m, m);
   const int64_t blocks = slots * col_tiles;
   BUX_CHECK(blocks < (1LL << 31), "bux_bf16_grouped_rows_f32: too many tiles");
@@ -899,32 +938,68 @@ extern "C" int bux_bf16_grouped_rows_f32(const float* x, const float* w, int w_t
   return launched("rows_f32_kernel");
 }
 
-extern "C" int bux_bf16_grouped_contract_f32(const float* x, const float* dy, const int32_t* sizes,
+extern "C" int bux_bf16_grouped_rows_f32(const float* x, const float* w, int w_transposed,
+                                         const int32_t* sizes, int32_t groups, int64_t m,
+                                         int64_t n, int64_t k, float* y, void* workspace,
+                                         size_t workspace_bytes, void* stream) {
+  using namespace bux;
+  clear_error();
+  BUX_CHECK(sizes != nullptr, "bux_bf16_grouped_rows_f32: NULL buffer");
+  return rows_f32_on(x, w, w_transposed, sizes, groups, m, n, k, y, workspace, workspace_bytes, stream);
+}
+
+extern "C" int bux_bf16_grouped_rows_listed_f32(const float* x, const float* w, int w_transposed,
+                                         int32_t groups, int64_t m,
+                                         int64_t n, int64_t k, float* y, void* list,
+                                         size_t list_bytes, void* stream) {
+  bux::clear_error();
+  return rows_f32_on(x, w, w_transposed, nullptr, groups, m, n, k, y, list, list_bytes, stream);
+}
+
+static int contract_f32_on(const float* x, const float* dy, const int32_t* sizes,
                                              int32_t groups, int64_t m, int64_t k, int64_t n,
                                              float* dw, void* workspace, size_t workspace_bytes,
                                              void* stream) {
   using namespace bux;
-  clear_error();
   BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS,
             "bux_bf16_grouped_contract_f32: groups=%d outside [1, %d]", groups, MAX_GROUPS);
   BUX_CHECK(m >= 0 && n > 0 && k > 0,
             "bux_bf16_grouped_contract_f32: bad shape m=%lld k=%lld n=%lld", (long long)m,
             (long long)k, (long long)n);
   BUX_CHECK(m < INT32_MAX, "bux_bf16_grouped_contract_f32: m=%lld rows", (long long)m);
-  BUX_CHECK(sizes && dw && (m == 0 || (x && dy)), "bux_bf16_grouped_contract_f32: NULL buffer");
+  BUX_CHECK(dw && (m == 0 || (x && dy)), "bux_bf16_grouped_contract_f32: NULL buffer");
   const size_t need = bux_bf16_grouped_contract_workspace_size(groups);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(BUX_E_WORKSPACE,
                 "bux_bf16_grouped_contract_f32: workspace of %zu bytes, %zu needed",
                 workspace_bytes, need);
   hipStream_t s = as_stream(stream);
-  hipLaunchKernelGGL(prologue_kernel, dim3(1), dim3(THREADS), 0, s, sizes, groups, 0, 0, 1,
-                     starts_in(workspace), nullptr, header_in(workspace), m, nullptr);
-  if (int rc = launched("prologue_kernel")) return rc;
+  if (sizes) {
+    hipLaunchKernelGGL(prologue_kernel, dim3(1), dim3(THREADS), 0, s, sizes, groups, 0, 0, 1,
+                       starts_in(workspace), nullptr, header_in(workspace), m, nullptr);
+    if (int rc = launched("prologue_kernel")) return rc;
+  }
   const int64_t k_tiles = ceil_div(k, BM), col_tiles = ceil_div(n, ANY_BN);
   const int64_t blocks = static_cast<int64_t>(groups) * k_tiles * col_tiles;
   BUX_CHECK(blocks < (1LL << 31), "bux_bf16_grouped_contract_f32: too many tiles");
   hipLaunchKernelGGL(contract_f32_kernel, dim3(static_cast<unsigned>(blocks)), dim3(THREADS), 0, s,
                      x, dy, groups, m, k, n, starts_in(workspace), k_tiles, col_tiles, dw);
   return launched("contract_f32_kernel");
+}
+
+extern "C" int bux_bf16_grouped_contract_f32(const float* x, const float* dy, const int32_t* sizes,
+                                             int32_t groups, int64_t m, int64_t k, int64_t n,
+                                             float* dw, void* workspace, size_t workspace_bytes,
+                                             void* stream) {
+  using namespace bux;
+  clear_error();
+  BUX_CHECK(sizes != nullptr, "bux_bf16_grouped_contract_f32: NULL buffer");
+  return contract_f32_on(x, dy, sizes, groups, m, k, n, dw, workspace, workspace_bytes, stream);
+}
+
+extern "C" int bux_bf16_grouped_contract_listed_f32(const float* x, const float* dy, int32_t groups, int64_t m, int64_t k, int64_t n,
+                                             float* dw, void* list, size_t list_bytes,
+                                             void* stream) {
+  bux::clear_error();
+  return contract_f32_on(x, dy, nullptr, groups, m, k, n, dw, list, list_bytes, stream);
 }

@@ -521,7 +521,7 @@ class Saved(NamedTuple):
     h_m: Tiled | None  # h^T along the rows (wgrad of down in MXFP8)
     down_n: Tiled | None  # each W_down along n (dgrad of down in MXFP8)
     rows: torch.Tensor | None  # the picks' rows (wgrad of up in bfloat16)
-    tiles: grouped_mxfp8.TileList | None = None  # the MXFP8 GEMMs' tile list, made once
+    tiles: grouped_mxfp8.TileList | None = None  # the GEMMs' tile list, made once
     passes: tuple[bool, bool, bool] = (True, True, True)  # (fprop, dgrad, wgrad) in MXFP8
     y: torch.Tensor | None = None  # with an expert norm: the down GEMM's rows (m, d)
 
@@ -602,9 +602,11 @@ def experts_forward(
         quantized.check(fmt, up, down)
     height = grouped_mxfp8.whole(m)
     with span("permute"):
-        # with one tile list for the step's six GEMMs: a of `height` rows, outputs of m
-        s, row_weights, listed = sort_for_layer(idx, e, weights,
-                                                height if fprop or dgrad or wgrad else None)
+        # with one tile list for the step's six GEMMs: in MXFP8 a of `height` rows and
+        # outputs of m, in "compute" both of m (a pass outside MXFP8 makes its own)
+        mx = fprop or dgrad or wgrad
+        s, row_weights, listed = sort_for_layer(idx, e, weights, height if mx else m)
+        plain = None if mx else listed
         filled = s.filled
     up2 = up.reshape(e, d, f * p)
     tiles = fmt == "mxfp8_2d"
@@ -641,7 +643,7 @@ def experts_forward(
                     x_k, up_k, s.sizes, dt, height=m, tiles=listed,
                     bias=None if up_bias is None else up_bias.reshape(e, f * p).contiguous())
             else:
-                projected = grouped.dot(rows, up2, s.sizes)
+                projected = grouped.dot(rows, up2, s.sizes, tiles=plain)
         if up_bias is not None and not fprop:
             with span("up bias"):
                 add_expert_bias(projected, up_bias.reshape(e, f * p), s.offsets)
@@ -666,7 +668,7 @@ def experts_forward(
         if fprop:
             y = grouped_mxfp8.rows(h_k, down_k, s.sizes, dt, height=m, tiles=listed)
         else:
-            y = grouped.dot(h, down, s.sizes)
+            y = grouped.dot(h, down, s.sizes, tiles=plain)
     y_rows = None
     if norm is not None:
         with span("expert norm"):
@@ -721,6 +723,7 @@ def experts_backward(saved: Saved, dy: torch.Tensor, up: torch.Tensor, down: tor
     if (fprop or dgrad or wgrad) != (fmt in MX_FORMATS):
         raise ValueError(f"experts_backward: fmt {fmt!r} is not the forward's")
     height = grouped_mxfp8.whole(m)
+    plain = None if fprop or dgrad or wgrad else saved.tiles
     dy_n = dy_m = dp_n = dp_m = dy_rows = None
     grads = {}
     if norm is not None:
@@ -765,12 +768,12 @@ def experts_backward(saved: Saved, dy: torch.Tensor, up: torch.Tensor, down: tor
             if dgrad:
                 dh = grouped_mxfp8.rows(dy_n, saved.down_n, s.sizes, dt, height=m, tiles=saved.tiles)
             else:
-                dh = grouped.dot(dy_rows, down, s.sizes, transposed=True)
+                dh = grouped.dot(dy_rows, down, s.sizes, transposed=True, tiles=plain)
     with span("down wgrad"):
         if wgrad:
             d_down = grouped_mxfp8.contract(saved.h_m, dy_m, s.sizes, dt, tiles=saved.tiles)
         else:
-            d_down = grouped.weight_grad(saved.h, dy_rows, s.sizes)
+            d_down = grouped.weight_grad(saved.h, dy_rows, s.sizes, tiles=plain)
     if twin:
         pass
     elif dgrad or wgrad:
@@ -789,12 +792,12 @@ def experts_backward(saved: Saved, dy: torch.Tensor, up: torch.Tensor, down: tor
         if dgrad:
             dx = grouped_mxfp8.rows(dp_n, saved.up_n, s.sizes, dt, height=m, tiles=saved.tiles)
         else:
-            dx = grouped.dot(dp, up2, s.sizes, transposed=True)
+            dx = grouped.dot(dp, up2, s.sizes, transposed=True, tiles=plain)
     with span("up wgrad"):
         if wgrad:
             d_up = grouped_mxfp8.contract(saved.x_m, dp_m, s.sizes, dt, tiles=saved.tiles)
         else:
-            d_up = grouped.weight_grad(saved.rows, dp, s.sizes)
+            d_up = grouped.weight_grad(saved.rows, dp, s.sizes, tiles=plain)
     if up_bias is not None:
         with span("up bias grad"):
             grads["up_bias"] = expert_sums(dp, s.offsets).view(e, f, p)

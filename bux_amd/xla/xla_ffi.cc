@@ -268,6 +268,34 @@ XLA_FFI_DEFINE_HANDLER_SYMBOL(BuxBf16Contract, Bf16Contract,
                               ffi::Ffi::Bind().Ctx<Stream>().Arg<In>().Arg<In>().Arg<In>()
                                   .Ret<In>().Ret<In>());
 
+static ffi::Error Bf16RowsListed(hipStream_t s, In x, In w, In list, int64_t transposed, Out y) {
+  if (f32(x))
+    return status(bux_bf16_grouped_rows_listed_f32(
+        at<const float>(x), at<const float>(w), static_cast<int>(transposed),
+        static_cast<int32_t>(dim(w, 0)), dim(x, 0), dim(y, 1), dim(x, 1), at<float>(y),
+        at<void>(list), list.size_bytes(), s));
+  return status(bux_bf16_grouped_rows_listed(
+      at<const uint16_t>(x), at<const uint16_t>(w), static_cast<int>(transposed),
+      static_cast<int32_t>(dim(w, 0)), dim(x, 0), dim(y, 1), dim(x, 1), at<uint16_t>(y),
+      at<void>(list), list.size_bytes(), s));
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(BuxBf16RowsListed, Bf16RowsListed,
+                              ffi::Ffi::Bind().Ctx<Stream>().Arg<In>().Arg<In>().Arg<In>()
+                                  .Attr<int64_t>("transposed").Ret<In>());
+
+static ffi::Error Bf16ContractListed(hipStream_t s, In x, In dy, In list, Out dw) {
+  if (f32(x))
+    return status(bux_bf16_grouped_contract_listed_f32(
+        at<const float>(x), at<const float>(dy), static_cast<int32_t>(dim(dw, 0)), dim(x, 0),
+        dim(x, 1), dim(dy, 1), at<float>(dw), at<void>(list), list.size_bytes(), s));
+  return status(bux_bf16_grouped_contract_listed(
+      at<const uint16_t>(x), at<const uint16_t>(dy), static_cast<int32_t>(dim(dw, 0)), dim(x, 0),
+      dim(x, 1), dim(dy, 1), at<uint16_t>(dw), at<void>(list), list.size_bytes(), s));
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(BuxBf16ContractListed, Bf16ContractListed,
+                              ffi::Ffi::Bind().Ctx<Stream>().Arg<In>().Arg<In>().Arg<In>()
+                                  .Ret<In>());
+
 // --- a-2, a-3: the token path's gathers and sums ---------------------------------------
 
 static ffi::Error TokenRows(hipStream_t s, In z, In order, int64_t k, Out rows) {

@@ -299,6 +299,19 @@ int bux_bf16_grouped_rows_f32(const float* x, const float* w, int w_transposed,
 int bux_bf16_grouped_contract_f32(const float* x, const float* dy, const int32_t* sizes,
                                   int32_t groups, int64_t m, int64_t k, int64_t n, float* dw,
                                   void* workspace, size_t workspace_bytes, void* stream);
+/* The _listed forms take a tile list in place of the sizes and their own prologue: made by
+ * bux_mx_grouped_tiles or bux_moe_permute_layer for m rows into a height of m (rows), or any
+ * list of the same groups (contract); refused as bux_mx_grouped_rows_listed refuses. */
+int bux_bf16_grouped_rows_listed(const uint16_t* x, const uint16_t* w, int w_transposed, int32_t
+    groups, int64_t m, int64_t n, int64_t k, uint16_t* y, void* list, size_t list_bytes, void*
+    stream);
+int bux_bf16_grouped_contract_listed(const uint16_t* x, const uint16_t* dy, int32_t groups,
+    int64_t m, int64_t k, int64_t n, uint16_t* dw, void* list, size_t list_bytes, void* stream);
+int bux_bf16_grouped_rows_listed_f32(const float* x, const float* w, int w_transposed, int32_t
+    groups, int64_t m, int64_t n, int64_t k, float* y, void* list, size_t list_bytes, void*
+    stream);
+int bux_bf16_grouped_contract_listed_f32(const float* x, const float* dy, int32_t groups,
+    int64_t m, int64_t k, int64_t n, float* dw, void* list, size_t list_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------------
  * a-2 / a-3. The token path's gathers and sums.

@@ -1,0 +1,34 @@
+"""The "compute" GEMMs on a tile list made once give the bits of those that make their own,
+in bfloat16 and float32, on the tiled and the any-shape kernels, and refuse a list made for
+other dimensions."""
+
+import numpy as np
+import pytest
+import torch
+
+from tests._util import announce
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("sizes,m,k,n", [([300, 0, 77, 500], 900, 64, 264), ([5, 0, 3], 10, 45, 37),
+                                         ([0, 0], 64, 32, 32), ([513] + [3] * 40, 700, 128, 128)])
+def test_listed_gemms_are_the_others(lib, sizes, m, k, n, dtype):
+    from bux_amd import grouped, grouped_mxfp8
+    g = torch.Generator(device="cuda").manual_seed(120)
+    gs = torch.tensor(sizes, dtype=torch.int32, device="cuda")
+    x, w, dy = (torch.randn(*s, generator=g, device="cuda").to(dtype)
+                for s in ((m, k), (len(sizes), k, n), (m, n)))
+    tiles = grouped_mxfp8.tiles_of(gs, m, m)
+    announce("listed compute GEMMs", sizes[:4], m, k, n, dtype)
+    pairs = [(grouped.dot(x, w, gs), grouped.dot(x, w, gs, tiles=tiles)),
+             (grouped.dot(dy, w, gs, transposed=True), grouped.dot(dy, w, gs, transposed=True, tiles=tiles)),
+             (grouped.weight_grad(x, dy, gs), grouped.weight_grad(x, dy, gs, tiles=tiles))]
+    torch.cuda.synchronize()
+    for own, listed in pairs:
+        assert torch.equal(own, listed)
+    with pytest.raises(ValueError):
+        grouped.dot(x, w, gs, tiles=grouped_mxfp8.tiles_of(gs, m + 128, m))
+    with pytest.raises(ValueError):
+        grouped.weight_grad(x, dy, gs, tiles=grouped_mxfp8.tiles_of(torch.cat([gs, gs]), m, m))
