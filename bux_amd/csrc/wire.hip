@@ -28,7 +28,6 @@ namespace bux {
 namespace {
 
 constexpr int THREADS = 256;
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void unpack8(const uint4& r, float* v) {
   const uint32_t w[4] = {r.x, r.y, r.z, r.w};
@@ -160,13 +159,13 @@ __global__ __launch_bounds__(THREADS) void unpack_kernel(const uint8_t* __restri
       // v_cvt_pk_f32_fp8: two E4M3 codes (the word's low or high half) to two floats
       const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(w[i]), false);
       const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(w[i]), true);
-      o[2 * i] = pack_bf16x2(lo[0] * scale, lo[1] * scale);
-      o[2 * i + 1] = pack_bf16x2(hi[0] * scale, hi[1] * scale);
+      o[2 * i] = static_cast<uint32_t>(f32_to_bf16(lo[0] * scale)) |
+                 (static_cast<uint32_t>(f32_to_bf16(lo[1] * scale)) << 16);
+      o[2 * i + 1] = static_cast<uint32_t>(f32_to_bf16(hi[0] * scale)) |
+                     (static_cast<uint32_t>(f32_to_bf16(hi[1] * scale)) << 16);
     }
-    // non-temporal: config 3's 131072 rows 150 us with ordinary stores, 133 so, 132 with
-    // the hardware's rounding
-    __builtin_nontemporal_store(u32x4{o[0], o[1], o[2], o[3]},
-                                reinterpret_cast<u32x4*>(out + u[j].row * d + 32 * u[j].b + 8 * u[j].q));
+    *reinterpret_cast<uint4*>(out + u[j].row * d + 32 * u[j].b + 8 * u[j].q) =
+        make_uint4(o[0], o[1], o[2], o[3]);
   }
 }
 
