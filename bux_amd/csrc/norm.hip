@@ -18,8 +18,8 @@
 // groups: the picks outside the experts, whose weights the layer zeroes) give 0.
 //
 // Forward: a workgroup a row, the row in registers (d <= 8192: 8 values a thread a 2048
-// chunk), block sums through LDS. Backward: a workgroup takes rows_a_block rows one after
-// another, each thread the same columns of every row, so that it adds its columns' gain and
+// chunk), block sums through LDS. Backward: a workgroup of backward_blocks takes an even share
+// of the rows one after another, each thread the same columns of every row, so that it adds its columns' gain and
 // bias gradients over the rows in registers; one float32 partial a workgroup and column
 // goes to the workspace, and norm_params_kernel adds the partials in a fixed order.
 //
@@ -42,10 +42,12 @@ constexpr int VEC = 8;
 constexpr int MAX_CHUNKS = 4;  // d <= MAX_CHUNKS * THREADS * VEC = 8192
 constexpr int MAX_ROWS = 64;   // rows a backward workgroup, at most
 
-// The rows a backward workgroup takes of m: about 1024 workgroups (4 a CU).
-int64_t rows_a_block(int64_t m) {
-  const int64_t r = (m + 1023) / 1024;
-  return r < 1 ? 1 : (r < MAX_ROWS ? r : MAX_ROWS);
+// The backward's workgroups over m rows: a row each up to 1024 (4 a CU), then 1024 until
+// they take MAX_ROWS each. It never falls as m grows: a workspace for the most rows a caller
+// has serves fewer too.
+int64_t backward_blocks(int64_t m) {
+  const int64_t most = m < 1024 ? m : 1024, least = ceil_div(m, MAX_ROWS);
+  return most > least ? most : least;
 }
 
 // The sum of v over the workgroup (256 threads); `red` 4 floats of LDS. Every thread
@@ -180,12 +182,13 @@ __global__ __launch_bounds__(THREADS) void norm_forward_kernel(
   }
 }
 
-// A workgroup takes rows [blockIdx.x rows, + rows): dv and the weights' gradient a row,
-// and its columns' gain and bias gradients summed over its rows into partials[2][block][d].
+// A workgroup takes `rows` rows, the first `longer` workgroups one more: dv and the weights'
+// gradient a row, and its columns' gain and bias gradients summed over its rows into
+// partials[2][block][d].
 template <typename T, int C>
 __global__ __launch_bounds__(THREADS) void norm_backward_kernel(
     const T* __restrict__ dy, const int32_t* __restrict__ index, int32_t index_div,
-    int64_t sources, const T* __restrict__ y, int64_t m, int64_t d, int64_t rows, NormArgs<T> a,
+    int64_t sources, const T* __restrict__ y, int64_t rows, int64_t longer, int64_t d, NormArgs<T> a,
     const T* __restrict__ weights, T* __restrict__ dv, T* __restrict__ d_weights,
     float* __restrict__ partials) {
   // Each product rounds before it is added, as the reference's ops do (no FMA contraction).
@@ -197,8 +200,9 @@ __global__ __launch_bounds__(THREADS) void norm_backward_kernel(
   for (int i = 0; i < C; ++i)
 #pragma unroll
     for (int j = 0; j < VEC; ++j) d_gain.v[i][j] = d_bias.v[i][j] = 0.0f;
-  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rows;
-  for (int64_t r = r0; r < r0 + rows && r < m; ++r) {
+  const int64_t b = blockIdx.x;
+  const int64_t r0 = b * rows + (b < longer ? b : longer), end = r0 + rows + (b < longer ? 1 : 0);
+  for (int64_t r = r0; r < end; ++r) {
     const int32_t e = expert_of(a.offsets, a.experts, r);
     T* o = dv + r * d;
     if (e < 0) {  // uniform: the whole workgroup's row
@@ -370,7 +374,7 @@ int norm_forward(const char* name, const T* y, int64_t m, int64_t d, const T* do
 }
 
 size_t backward_workspace(int64_t m, int64_t d) {
-  return static_cast<size_t>(2 * ceil_div(m, rows_a_block(m)) * d) * sizeof(float);
+  return static_cast<size_t>(2 * backward_blocks(m) * d) * sizeof(float);
 }
 
 template <typename T>
@@ -391,13 +395,13 @@ int norm_backward(const char* name, const T* dy, const int32_t* index, int32_t i
     return fail(BUX_E_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", name, workspace_bytes,
                 need);
   hipStream_t s = as_stream(stream);
-  const int64_t rows = rows_a_block(m), blocks = ceil_div(m, rows);
+  const int64_t blocks = backward_blocks(m);
   if (m > 0) {
     BUX_CHECK(dy && y && weights && dv && d_weights, "%s: NULL buffer", name);
     with_chunks(d, [&](auto c) {
       hipLaunchKernelGGL((norm_backward_kernel<T, decltype(c)::value>),
                          dim3(static_cast<unsigned>(blocks)), dim3(THREADS), 0, s, dy, index,
-                         index_div, sources, y, m, d, rows, a, weights, dv, d_weights,
+                         index_div, sources, y, m / blocks, m % blocks, d, a, weights, dv, d_weights,
                          static_cast<float*>(workspace));
     });
     if (int rc = launched("norm_backward_kernel")) return rc;

@@ -376,3 +376,13 @@ def test_the_layers_sort_rejects_bad_arguments(lib):
     assert sort(m=64, height=96) == 1 and "100 picks" in _msg(lib)  # a list shorter than the picks
     assert sort(list_bytes=64) == 2 and "list" in _msg(lib)
     assert sort(ws=4) == 2 and "workspace" in _msg(lib)
+
+
+def test_the_norm_backwards_workspace_never_falls_as_rows_grow(lib):
+    """One sized for a caller's largest m serves every smaller one, around the rows at
+    which its workgroups take one more row each and at which they take their most."""
+    for d in (8, 2056, 7168):
+        sizes = [lib.bux_expert_norm_backward_workspace_size(m, d)
+                 for m in [*range(0, 4200), *range(65000, 66700), 131072, 1 << 20]]
+        assert sizes == sorted(sizes)
+        assert sizes[0] == 0 and sizes[1] == 8 * d

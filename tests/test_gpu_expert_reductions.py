@@ -61,3 +61,27 @@ def test_expert_sums(lib, sizes, width, dtype):
         start += size
         err = (got[e].double() - part.sum(0)).abs()
         assert bool((err <= size * 2.0**-24 * part.abs().sum(0)).all())
+
+
+@pytest.mark.parametrize("m,d", [(1023, 256), (1024, 256), (1025, 256), (2049, 2056), (65537, 8)])
+def test_norm_gradients_of_every_row(lib, m, d):
+    """dv and the weights' gradients are a row's own, whichever workgroup takes it: the bits
+    of calls on parts of the rows."""
+    from bux_amd import moe
+    g = torch.Generator(device="cuda").manual_seed(92)
+    y, dy, w = (torch.randn(*s, generator=g, device="cuda") for s in ((m, d), (m, d), (m,)))
+    scale = torch.randn(d, generator=g, device="cuda")
+    norm = moe.ExpertNorm("rmsnorm")
+
+    def backward(lo, hi):
+        order = torch.arange(hi - lo, dtype=torch.int32, device="cuda")
+        return moe.expert_norm_backward(dy[lo:hi], order, 1, y[lo:hi], _offsets([hi - lo]), norm, scale,
+                                        None, w[lo:hi])[:2]
+
+    announce("norm gradients of every row", m, d)
+    got = backward(0, m)
+    cuts = [0, *range(500, m, 500), m]
+    parts = [backward(lo, hi) for lo, hi in zip(cuts, cuts[1:])]
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert torch.equal(got[i], torch.cat([p[i] for p in parts]))
