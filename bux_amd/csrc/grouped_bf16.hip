@@ -390,12 +390,13 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
 
 // contract: A = x, B = dy, both MN-major over the rows (K).
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void contract_kernel(
-    Operand A, Operand B, int32_t groups, int32_t d, int32_t f, const int32_t* __restrict__ starts,
-    int32_t d_tiles, int32_t f_tiles, uint16_t* __restrict__ dw) {
+    Operand A, Operand B, int32_t groups, int32_t m, int32_t d, int32_t f,
+    const int32_t* __restrict__ starts, int32_t d_tiles, int32_t f_tiles,
+    uint16_t* __restrict__ dw) {
   extern __shared__ __align__(16) uint8_t smem[];
   if (!list_fits(starts, groups, -1, 0)) return;
   Lds& lds = *reinterpret_cast<Lds*>(smem);
-  const ContractTiles list{starts, d, f, d_tiles, f_tiles, BK};
+  const ContractTiles list{starts, d, f, d_tiles, f_tiles, BK, m};
   const int32_t count = groups * d_tiles * f_tiles;
   run_tiles<Bf16<false, false>>(list, count, A, B, lds, Out{dw, f});
 }
@@ -855,7 +856,8 @@ static int contract_on(const uint16_t* x, const uint16_t* dy, const int32_t* siz
     return fail(BUX_E_WORKSPACE, "bux_bf16_grouped_contract: workspace of %zu bytes, %zu needed",
                 workspace_bytes, need);
   hipStream_t s = as_stream(stream);
-  // the starts capped at the contract's K (m rows), as the rows GEMM caps them at its rows
+  // the starts capped at the contract's K (m rows), as the rows GEMM caps them at its rows;
+  // a list's may reach further: the kernels cap them again
   if (sizes) {
     hipLaunchKernelGGL(prologue_kernel, dim3(1), dim3(THREADS), 0, s, sizes, groups, 0, 0, 1,
                        starts_in(workspace), nullptr, header_in(workspace), m, nullptr);
@@ -879,8 +881,9 @@ static int contract_on(const uint16_t* x, const uint16_t* dy, const int32_t* siz
   if (int rc = grid_for(tiles, &blocks)) return rc;
   if (int rc = allow_lds(contract_kernel, sizeof(Lds), "bf16 contract_kernel")) return rc;
   hipLaunchKernelGGL(contract_kernel, dim3(blocks), dim3(THREADS), sizeof(Lds), s, A, B, groups,
-                     static_cast<int32_t>(k), static_cast<int32_t>(n), starts_in(workspace),
-                     static_cast<int32_t>(d_tiles), static_cast<int32_t>(f_tiles), dw);
+                     static_cast<int32_t>(m), static_cast<int32_t>(k), static_cast<int32_t>(n),
+                     starts_in(workspace), static_cast<int32_t>(d_tiles),
+                     static_cast<int32_t>(f_tiles), dw);
   return launched("bf16 contract_kernel");
 }
 

@@ -805,7 +805,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
   extern __shared__ __align__(16) uint8_t smem[];
   if (!list_fits(starts, groups, -1, 0)) return;
   Lds& lds = *reinterpret_cast<Lds*>(smem);
-  const ContractTiles list{starts, A.rows, B.rows, d_tiles, f_tiles, BK};
+  const ContractTiles list{starts, A.rows, B.rows, d_tiles, f_tiles, BK, A.k};
   const int32_t count = groups * d_tiles * f_tiles;
   run_tiles<MxOf<W>>(list, count, A, B, lds, Plain<T>{dw, B.rows});
 }

@@ -175,7 +175,7 @@ __device__ __forceinline__ Turns turns(int32_t count) {
   return Turns{lo + static_cast<int32_t>(blockIdx.x / 8), hi, static_cast<int32_t>(gridDim.x / 8)};
 }
 
-__device__ __forceinline__ int32_t smaller(int32_t a, int32_t b) { return a < b ? a : b; }
+__host__ __device__ __forceinline__ int32_t smaller(int32_t a, int32_t b) { return a < b ? a : b; }
 
 // One output tile's work: C[r][c] = sum over K steps [ks_begin, ks_begin + n) of
 // A[a_row0 + r] . B[b_row0 + c] (B of `group`), the K positions outside [mlo, mhi)
@@ -255,17 +255,18 @@ struct StartedTiles {
 };
 
 // The contract GEMM's tiles: each group's d x f output in 256 x 256 tiles; K is the
-// rows of the operands, `step` of them a K step, and a group's sum takes its own rows
-// [starts[g], starts[g + 1]) only.
+// operands' m rows, `step` of them a K step, and a group's sum takes its own rows
+// [starts[g], starts[g + 1]) only, those below m: the starts may be a list's that was made
+// for more rows, and a step past m has an offset outside the 32 bits the host checked.
 struct ContractTiles {
   static constexpr bool HALVES = false;
   const int32_t* starts;
-  int32_t d, f, d_tiles, f_tiles, step;
-  __device__ bool job(int32_t id, Job& j) const {
+  int32_t d, f, d_tiles, f_tiles, step, m;
+  __host__ __device__ bool job(int32_t id, Job& j) const {
     const int32_t per_group = d_tiles * f_tiles;
     const int32_t g = id / per_group, rest = id % per_group;
     const int32_t row0 = (rest / f_tiles) * BM, col0 = (rest % f_tiles) * BN;
-    const int32_t start = starts[g], end = starts[g + 1];
+    const int32_t start = smaller(starts[g], m), end = smaller(starts[g + 1], m);
     j.a_row0 = row0;
     j.b_row0 = col0;
     j.group = 0;

@@ -54,7 +54,8 @@ def dot(x: torch.Tensor, w: torch.Tensor, sizes: torch.Tensor, transposed: bool 
 def weight_grad(x: torch.Tensor, dy: torch.Tensor, sizes: torch.Tensor,
                 tiles: TileList | None = None) -> torch.Tensor:
     """Return ``x[rows of g]^T dy[rows of g]`` for each group g, (g, k, n), in x's dtype
-    (bfloat16 or float32, dy the same). tiles: a tile list of the same sizes, as `dot`'s."""
+    (bfloat16 or float32, dy the same). tiles: a tile list of the same sizes, as `dot`'s,
+    or of more rows: those past x's add nothing."""
     require(x, dy, sizes)
     f32 = _f32("weight_grad", x, dy)
     m, k = x.shape

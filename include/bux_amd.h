@@ -301,7 +301,8 @@ int bux_bf16_grouped_contract_f32(const float* x, const float* dy, const int32_t
                                   void* workspace, size_t workspace_bytes, void* stream);
 /* The _listed forms take a tile list in place of the sizes and their own prologue: made by
  * bux_mx_grouped_tiles or bux_moe_permute_layer for m rows into a height of m (rows), or any
- * list of the same groups (contract); refused as bux_mx_grouped_rows_listed refuses. */
+ * list of the same groups (contract, the MXFP8 one too: of a list for more rows than m it
+ * takes those below m); refused as bux_mx_grouped_rows_listed refuses. */
 int bux_bf16_grouped_rows_listed(const uint16_t* x, const uint16_t* w, int w_transposed, int32_t
     groups, int64_t m, int64_t n, int64_t k, uint16_t* y, void* list, size_t list_bytes, void*
     stream);

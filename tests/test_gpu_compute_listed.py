@@ -32,3 +32,28 @@ def test_listed_gemms_are_the_others(lib, sizes, m, k, n, dtype):
         grouped.dot(x, w, gs, tiles=grouped_mxfp8.tiles_of(gs, m + 128, m))
     with pytest.raises(ValueError):
         grouped.weight_grad(x, dy, gs, tiles=grouped_mxfp8.tiles_of(torch.cat([gs, gs]), m, m))
+
+
+@pytest.mark.parametrize("kind", ["bfloat16", "float32", "any shape", "mxfp8"])
+def test_a_contract_on_a_list_of_more_rows(lib, kind):
+    """A contract takes the rows below its own m of a list made for more: the bits of the
+    starts that its own prologue caps."""
+    from bux_amd import grouped, grouped_mxfp8
+    g = torch.Generator(device="cuda").manual_seed(121)
+    m, d, f = 384, 72, 264
+    if kind == "any shape":
+        d, f = 45, 37
+    gs = torch.tensor([100, 0, 250, 700, 5], dtype=torch.int32, device="cuda")
+    longer = grouped_mxfp8.tiles_of(gs, 2048, 2048)
+    dtype = torch.float32 if kind == "float32" else torch.bfloat16
+    announce("contract on a longer list", kind)
+    if kind == "mxfp8":
+        x, dy = (torch.randn(m, c, generator=g, device="cuda").to(dtype) for c in (96, 160))
+        a, b = (grouped_mxfp8.quantized_twice(v, rows=False)[1] for v in (x, dy))
+        own, listed = (grouped_mxfp8.contract(a, b, gs, tiles=t) for t in (None, longer))
+    else:
+        x, dy = (torch.randn(m, c, generator=g, device="cuda").to(dtype) for c in (d, f))
+        own, listed = (grouped.weight_grad(x, dy, gs, tiles=t) for t in (None, longer))
+    torch.cuda.synchronize()
+    assert torch.equal(own, listed)
+    assert bool((own[:1] != 0).any()) and not own[4].any()
