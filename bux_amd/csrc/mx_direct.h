@@ -6,6 +6,13 @@
 
 namespace bux {
 
+// The first row of the kernel's block `i` of a tile that starts at `lo`: 64 bits, since a
+// tile of a list's last rows and its blocks past them reach beyond 2^31.
+constexpr int DIRECT_BLOCK = 32;  // rows a wave
+__host__ __device__ __forceinline__ int64_t direct_row(int32_t lo, uint32_t i) {
+  return lo + static_cast<int64_t>(DIRECT_BLOCK) * i;
+}
+
 // Whether a rows GEMM of `m` rows in `groups` groups, `n` columns, goes to
 // rows_direct_kernel.
 bool rows_direct(int64_t m, int32_t groups, int64_t n);

@@ -26,7 +26,6 @@ namespace {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 
-constexpr int BLOCK = 32;  // rows a wave
 constexpr int CB = 2;      // its blocks of 32 columns
 constexpr int D = 2;       // K pairs in flight
 
@@ -63,7 +62,7 @@ __global__ __launch_bounds__(64) void rows_direct_kernel(
   const int32_t id = blockIdx.x / col_blocks;
   if (id >= starts[groups + 1]) return;
   const Tile t = tiles[id];
-  const int32_t row0 = t.lo + static_cast<int32_t>(blockIdx.y) * BLOCK, end = smaller(t.hi, height);
+  const int64_t row0 = direct_row(t.lo, blockIdx.y), end = smaller(t.hi, height);
   if (row0 >= end) return;
   const int lane = threadIdx.x, half = lane >> 5, r32 = lane & 31;
   const int32_t col0 = (blockIdx.x % col_blocks) * 32 * CB;
@@ -73,7 +72,7 @@ __global__ __launch_bounds__(64) void rows_direct_kernel(
   const uint8_t* const bs = b_scales + static_cast<int64_t>(group) * n * (k / 32);
   const int64_t a_chunk = static_cast<int64_t>(a_rows) * 64, b_chunk = static_cast<int64_t>(n) * 64;
   // rows past an operand's are its last one's again, and not stored
-  const uint32_t ar = static_cast<uint32_t>(smaller(row0 + r32, a_rows - 1));
+  const uint32_t ar = static_cast<uint32_t>(row0 + r32 < a_rows ? row0 + r32 : a_rows - 1);
   uint32_t br[CB];
 #pragma unroll
   for (int j = 0; j < CB; ++j) br[j] = static_cast<uint32_t>(smaller(col0 + 32 * j + r32, n - 1));
@@ -147,7 +146,7 @@ __global__ __launch_bounds__(64) void rows_direct_kernel(
     if (p + D + i < pairs) multiply(in[i]);
 
   // lane l holds row l % 32, run g the columns 8 g + 4 (l / 32) .. + 3 of each block
-  const int32_t row = row0 + r32;
+  const int64_t row = row0 + r32;
   if (row >= end) return;
 #pragma unroll
   for (int j = 0; j < CB; ++j)
@@ -155,7 +154,7 @@ __global__ __launch_bounds__(64) void rows_direct_kernel(
     for (int g = 0; g < 4; ++g) {
       const int32_t col = col0 + 32 * j + 8 * g + 4 * half;
       if (col >= n) continue;  // n is a multiple of 4
-      T* at = y + static_cast<int64_t>(row) * n + col;
+      T* at = y + row * n + col;
       float c[4] = {acc[j][4 * g], acc[j][4 * g + 1], acc[j][4 * g + 2], acc[j][4 * g + 3]};
       if (bias != nullptr && pairs > 0) {  // the product rounded, then the sum
         const T* b = bias + static_cast<int64_t>(group) * n + col;
@@ -176,7 +175,7 @@ int launch_as(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b
   const int64_t col_blocks = ceil_div(n, 32 * CB);
   if (slots * col_blocks >= (1LL << 31)) return fail(BUX_E_ARGUMENT, "bux_mx_grouped_rows: too many tiles");
   const int64_t rows = m > height ? m : height;  // no tile holds more
-  const int64_t row_blocks = ceil_div(rows < BM ? rows : BM, BLOCK);
+  const int64_t row_blocks = ceil_div(rows < BM ? rows : BM, DIRECT_BLOCK);
   hipLaunchKernelGGL(rows_direct_kernel<T>,
                      dim3(static_cast<unsigned>(slots * col_blocks), static_cast<unsigned>(row_blocks)),
                      dim3(64), 0, s, a_values, a_scales, b_values, b_scales, static_cast<int32_t>(k),

@@ -134,12 +134,12 @@ __device__ __forceinline__ void write_list(const LayerOuts& o, const int32_t* of
     const int32_t g = base + static_cast<int32_t>(threadIdx.x);
     const int32_t lo = g <= num_experts ? offs[g] : 0;
     const int32_t hi = g < num_experts ? offs[g + 1] : g == num_experts && height > lo ? height : lo;
-    const int32_t count = (hi - lo + BM - 1) / BM;
+    const int32_t count = static_cast<int32_t>(tile_count(lo, hi));
     int32_t before;
     const int32_t total = block_exclusive<NT>(count, before, wave_sums);
     if (g <= num_experts) starts[g] = lo;
     for (int32_t j = 0; j < count && used + before + j < o.slots; ++j)
-      o.tiles[used + before + j] = Tile{g, lo + j * BM, smaller(hi, lo + (j + 1) * BM)};
+      o.tiles[used + before + j] = tile_at(g, lo, hi, j);
     used += total;
   }
   for (int64_t i = used + threadIdx.x; i < o.slots; i += NT) o.tiles[i] = Tile{0, 0, 0};

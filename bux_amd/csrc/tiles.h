@@ -32,6 +32,17 @@ struct Tile {
   int32_t group, lo, hi;
 };
 
+// The rows [lo, hi) of group g in tiles of BM from lo: how many, and tile j of them. In 64
+// bits, since a list may reach to 2^31 - 1 rows and a tile's end past them.
+__host__ __device__ __forceinline__ int64_t tile_count(int64_t lo, int64_t hi) {
+  return hi > lo ? (hi - lo + BM - 1) / BM : 0;
+}
+__host__ __device__ __forceinline__ Tile tile_at(int32_t g, int64_t lo, int64_t hi, int64_t j) {
+  const int64_t first = lo + j * BM;
+  return Tile{g, static_cast<int32_t>(first),
+              static_cast<int32_t>(hi < first + BM ? hi : first + BM)};
+}
+
 // --- the device-side prologue: group starts and the ragged tile list ----------------
 
 // Exclusive scan of data[0, n) (each >= 0) in LDS by one workgroup of THREADS lanes,
@@ -123,25 +134,20 @@ __global__ __launch_bounds__(THREADS) void prologue_kernel(const int32_t* __rest
     return a_starts != nullptr && g < groups ? static_cast<int64_t>(a_starts[g]) : starts[g];
   };
   // tiles of group g: from its first row rounded down to `align`
+  auto base_of = [&](int g) -> int64_t { return first(g) & ~static_cast<int64_t>(align - 1); };
   auto count_of = [&](int g) -> int64_t {
     const int64_t s = size_of(g);
-    if (s <= 0) return 0;
-    const int64_t start = first(g), base = start & ~static_cast<int64_t>(align - 1);
-    return (start + s - base + BM - 1) / BM;
+    return s > 0 ? tile_count(base_of(g), first(g) + s) : 0;
   };
   for (int g = t; g < all; g += THREADS) before[g] = static_cast<int32_t>(count_of(g));
   __syncthreads();
   const int32_t used = block_scan(before, all, partial, INT32_MAX);
   for (int g = t; g < all; g += THREADS) {
-    const int64_t s = size_of(g), start = first(g), end = start + s;
-    const int64_t base = start & ~static_cast<int64_t>(align - 1), count = count_of(g);
+    const int64_t base = base_of(g), end = first(g) + size_of(g), count = count_of(g);
     // The capped starts keep the counts within the slots; a tile past them would be
     // dropped, never written past the list.
-    for (int64_t j = 0; j < count && before[g] + j < slots; ++j) {
-      const int64_t lo = base + j * BM;
-      tiles[before[g] + j] = Tile{g, static_cast<int32_t>(lo),
-                                  static_cast<int32_t>(end < lo + BM ? end : lo + BM)};
-    }
+    for (int64_t j = 0; j < count && before[g] + j < slots; ++j)
+      tiles[before[g] + j] = tile_at(g, base, end, j);
   }
   for (int64_t i = used + t; i < slots; i += THREADS) tiles[i] = Tile{0, 0, 0};
   if (t == 0) starts_out[groups + 1] = used < slots ? used : static_cast<int32_t>(slots);

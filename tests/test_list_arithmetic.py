@@ -19,7 +19,7 @@ def run(tmp_path_factory):
 
     def go(body: str) -> list[list[int]]:
         src, exe = at / "main.hip", at / "main"
-        src.write_text('#include "tiles.h"\n#include <cstdio>\nusing namespace bux;\n'
+        src.write_text('#include "tiles.h"\n#include "mx_direct.h"\n#include <cstdio>\nusing namespace bux;\n'
                        f"int main() {{\n{body}\nreturn 0; }}\n")
         subprocess.run([HIPCC, "-x", "hip", "--offload-host-only", "-std=c++17", "-O1",
                         "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "bux_amd", "csrc"),
@@ -52,3 +52,27 @@ def test_a_contracts_steps_stay_below_its_rows(run, step):
                 assert bool(mask) == (lo % step != 0 or hi % step != 0)
             else:
                 assert n == 0
+
+
+def test_tiles_of_almost_2_31_rows(run):
+    """A group's tiles cover its rows once each, in order, up to the last row that 32 bits
+    hold; and the blocks of the last tile that reach past them stay past them."""
+    top = 2**31 - 1
+    cases = [(0, 0), (5, 4), (0, 1), (7, 263), (7, 264), (0, top), (top - 1, top), (top - 255, top),
+             (top - 256, top), (top - 700, top), (2**31 - 256, top)]
+    lines = run("\n".join(f"""
+  {{
+    const int64_t n = tile_count({lo}, {hi}), first = n > 4 ? n - 4 : 0;
+    for (int64_t j = first; j < n; ++j) {{
+      const Tile t = tile_at(3, {lo}, {hi}, j);
+      printf("%d %lld %lld %d %d %d\\n", {i}, (long long)n, (long long)j, t.group, t.lo, t.hi);
+    }}
+  }}""" for i, (lo, hi) in enumerate(cases)))
+    for i, (lo, hi) in enumerate(cases):
+        got = [line[1:] for line in lines if line[0] == i]
+        n = max(0, -(-(hi - lo) // 256))
+        assert got == [[n, j, 3, lo + 256 * j, min(hi, lo + 256 * (j + 1))]
+                       for j in range(max(0, n - 4), n)]
+    rows = run(f"""
+  for (uint32_t i = 0; i < 8; ++i) printf("%lld\\n", (long long)direct_row({top - 10}, i));""")
+    assert rows == [[top - 10 + 32 * i] for i in range(8)]
