@@ -53,6 +53,10 @@ ffi::Error status(int rc) {
   if (rc == 0) return ffi::Error::Success();
   return ffi::Error(ffi::ErrorCode::kInternal, std::string(bux_last_error()));
 }
+// An operand the C ABI takes as a pointer alone, whose length it cannot check.
+ffi::Error mismatch(const char* what) {
+  return ffi::Error(ffi::ErrorCode::kInvalidArgument, std::string(what));
+}
 int dtype_of(Out& y) { return y->element_type() == ffi::DataType::F32 ? BUX_F32 : BUX_BF16; }
 bool f32(const In& b) { return b.element_type() == ffi::DataType::F32; }
 
@@ -102,10 +106,16 @@ XLA_FFI_DEFINE_HANDLER_SYMBOL(BuxMoePermute, MoePermute,
                               ffi::Ffi::Bind().Ctx<Stream>().Arg<In>().Attr<int64_t>("num_experts")
                                   .Ret<In>().Ret<In>().Ret<In>().Ret<In>().Ret<In>());
 
-// weights: one a pick, bfloat16 or float32; list: bux_mx_grouped_tiles's buffer, or empty.
+// weights and row_weights: one a pick, bfloat16 or float32 both; list: bux_mx_grouped_tiles's
+// buffer, or empty.
 static ffi::Error MoePermuteLayer(hipStream_t s, In idx, In weights, int64_t num_experts,
                                   int64_t m, int64_t height, Out order, Out inverse, Out sizes,
                                   Out offsets, Out row_weights, Out list, Out ws) {
+  if (!(f32(weights) || weights.element_type() == ffi::DataType::BF16) ||
+      weights.element_count() != idx.element_count() ||
+      row_weights->element_type() != weights.element_type() ||
+      row_weights->element_count() != idx.element_count())
+    return mismatch("BuxMoePermuteLayer: weights and row_weights are one bfloat16 or float32 a pick");
   return status(bux_moe_permute_layer(
       at<const int32_t>(idx), static_cast<int64_t>(idx.element_count()),
       static_cast<int32_t>(num_experts), at<const void>(weights),
@@ -196,6 +206,9 @@ XLA_FFI_DEFINE_HANDLER_SYMBOL(BuxMxRowsListed, MxRowsListed,
 // bias [groups, n] in y's dtype.
 static ffi::Error MxRowsBiased(hipStream_t s, In av, In as, In bv, In bs, In list, In bias,
                                Out y) {
+  if (bias.element_type() != y->element_type() ||
+      static_cast<int64_t>(bias.element_count()) != dim(bv, 0) * dim(bv, 2))
+    return mismatch("BuxMxRowsBiased: bias is [groups, n] of y's dtype");
   return status(bux_mx_grouped_rows_biased(
       at<const uint8_t>(av), at<const uint8_t>(as), at<const uint8_t>(bv), at<const uint8_t>(bs),
       at<void>(list), list.size_bytes(), static_cast<int32_t>(dim(bv, 0)), dim(av, 1), dim(bv, 2),
