@@ -769,21 +769,20 @@ extern "C" size_t bux_bf16_grouped_rows_workspace_size(int32_t groups, int64_t m
 }
 
 // With `sizes` NULL, the workspace is a list already made of them (the _listed entry points).
-static int rows_on(const uint16_t* x, const uint16_t* w, int w_transposed,
-                                     const int32_t* sizes, int32_t groups, int64_t m, int64_t n,
-                                     int64_t k, uint16_t* y, void* workspace,
-                                     size_t workspace_bytes, void* stream) {
+static int rows_on(const char* name, const uint16_t* x, const uint16_t* w, int w_transposed,
+                   const int32_t* sizes, int32_t groups, int64_t m, int64_t n, int64_t k,
+                   uint16_t* y, void* workspace, size_t workspace_bytes, void* stream) {
   using namespace bux;
-  BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS, "bux_bf16_grouped_rows: groups=%d outside [1, %d]",
-            groups, MAX_GROUPS);
-  BUX_CHECK(m >= 0 && n > 0 && k > 0, "bux_bf16_grouped_rows: bad shape m=%lld n=%lld k=%lld",
-            (long long)m, (long long)n, (long long)k);
-  BUX_CHECK(m < INT32_MAX, "bux_bf16_grouped_rows: m=%lld rows", (long long)m);
-  BUX_CHECK(w && y && (m == 0 || x), "bux_bf16_grouped_rows: NULL buffer");
+  BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS, "%s: groups=%d outside [1, %d]", name, groups,
+            MAX_GROUPS);
+  BUX_CHECK(m >= 0 && n > 0 && k > 0, "%s: bad shape m=%lld n=%lld k=%lld", name, (long long)m,
+            (long long)n, (long long)k);
+  BUX_CHECK(m < INT32_MAX, "%s: m=%lld rows", name, (long long)m);
+  BUX_CHECK(w && y && (m == 0 || x), "%s: NULL buffer", name);
   const size_t need = bux_bf16_grouped_rows_workspace_size(groups, m);
   if (workspace == nullptr || workspace_bytes < need)
-    return fail(BUX_E_WORKSPACE, "bux_bf16_grouped_rows: workspace of %zu bytes, %zu needed",
-                workspace_bytes, need);
+    return fail(BUX_E_WORKSPACE, "%s: %s of %zu bytes, %zu needed", name,
+                sizes ? "workspace" : "list", workspace_bytes, need);
   if (m == 0) return BUX_OK;
   hipStream_t s = as_stream(stream);
   if (sizes) {
@@ -796,7 +795,7 @@ static int rows_on(const uint16_t* x, const uint16_t* w, int w_transposed,
   if (n % 8 != 0 || k % 8 != 0 || !fits(m, k) || !(w_transposed ? fits(n, k) : fits(k, n))) {
     const int64_t col_tiles = ceil_div(n, ANY_BN), slots = row_slots(groups, m, m);
     const int64_t blocks = slots * col_tiles;
-    BUX_CHECK(blocks < (1LL << 31), "bux_bf16_grouped_rows: too many tiles");
+    BUX_CHECK(blocks < (1LL << 31), "%s: too many tiles", name);
     if (w_transposed)
       hipLaunchKernelGGL(rows_any_kernel<true>, dim3(static_cast<unsigned>(blocks)), dim3(THREADS), 0, s,
                          x, w, groups, m, n, k, starts_in(workspace), tiles_in(workspace, groups),
@@ -822,17 +821,21 @@ extern "C" int bux_bf16_grouped_rows(const uint16_t* x, const uint16_t* w, int w
                                      int64_t k, uint16_t* y, void* workspace,
                                      size_t workspace_bytes, void* stream) {
   using namespace bux;
+  const char* const name = "bux_bf16_grouped_rows";
   clear_error();
-  BUX_CHECK(sizes != nullptr, "bux_bf16_grouped_rows: NULL buffer");
-  return rows_on(x, w, w_transposed, sizes, groups, m, n, k, y, workspace, workspace_bytes, stream);
+  BUX_CHECK(sizes != nullptr, "%s: NULL buffer", name);
+  return rows_on(name, x, w, w_transposed, sizes, groups, m, n, k, y, workspace, workspace_bytes,
+                 stream);
 }
 
-extern "C" int bux_bf16_grouped_rows_listed(const uint16_t* x, const uint16_t* w, int w_transposed,
-                                     int32_t groups, int64_t m, int64_t n,
-                                     int64_t k, uint16_t* y, void* list,
-                                     size_t list_bytes, void* stream) {
-  bux::clear_error();
-  return rows_on(x, w, w_transposed, nullptr, groups, m, n, k, y, list, list_bytes, stream);
+extern "C" int bux_bf16_grouped_rows_listed(const uint16_t* x, const uint16_t* w,
+                                            int w_transposed, int32_t groups, int64_t m,
+                                            int64_t n, int64_t k, uint16_t* y, void* list,
+                                            size_t list_bytes, void* stream) {
+  using namespace bux;
+  const char* const name = "bux_bf16_grouped_rows_listed";
+  clear_error();
+  return rows_on(name, x, w, w_transposed, nullptr, groups, m, n, k, y, list, list_bytes, stream);
 }
 
 extern "C" size_t bux_bf16_grouped_contract_workspace_size(int32_t groups) {
@@ -840,21 +843,20 @@ extern "C" size_t bux_bf16_grouped_contract_workspace_size(int32_t groups) {
   return starts_bytes(groups);  // the group starts alone: header, starts
 }
 
-static int contract_on(const uint16_t* x, const uint16_t* dy, const int32_t* sizes,
-                                         int32_t groups, int64_t m, int64_t k, int64_t n,
-                                         uint16_t* dw, void* workspace, size_t workspace_bytes,
-                                         void* stream) {
+static int contract_on(const char* name, const uint16_t* x, const uint16_t* dy,
+                       const int32_t* sizes, int32_t groups, int64_t m, int64_t k, int64_t n,
+                       uint16_t* dw, void* workspace, size_t workspace_bytes, void* stream) {
   using namespace bux;
-  BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS,
-            "bux_bf16_grouped_contract: groups=%d outside [1, %d]", groups, MAX_GROUPS);
-  BUX_CHECK(m >= 0 && n > 0 && k > 0, "bux_bf16_grouped_contract: bad shape m=%lld k=%lld n=%lld",
-            (long long)m, (long long)k, (long long)n);
-  BUX_CHECK(m < INT32_MAX, "bux_bf16_grouped_contract: m=%lld rows", (long long)m);
-  BUX_CHECK(dw && (m == 0 || (x && dy)), "bux_bf16_grouped_contract: NULL buffer");
+  BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS, "%s: groups=%d outside [1, %d]", name, groups,
+            MAX_GROUPS);
+  BUX_CHECK(m >= 0 && n > 0 && k > 0, "%s: bad shape m=%lld k=%lld n=%lld", name, (long long)m,
+            (long long)k, (long long)n);
+  BUX_CHECK(m < INT32_MAX, "%s: m=%lld rows", name, (long long)m);
+  BUX_CHECK(dw && (m == 0 || (x && dy)), "%s: NULL buffer", name);
   const size_t need = bux_bf16_grouped_contract_workspace_size(groups);
   if (workspace == nullptr || workspace_bytes < need)
-    return fail(BUX_E_WORKSPACE, "bux_bf16_grouped_contract: workspace of %zu bytes, %zu needed",
-                workspace_bytes, need);
+    return fail(BUX_E_WORKSPACE, "%s: %s of %zu bytes, %zu needed", name,
+                sizes ? "workspace" : "list", workspace_bytes, need);
   hipStream_t s = as_stream(stream);
   // the starts capped at the contract's K (m rows), as the rows GEMM caps them at its rows;
   // a list's may reach further: the kernels cap them again
@@ -866,14 +868,14 @@ static int contract_on(const uint16_t* x, const uint16_t* dy, const int32_t* siz
   if (n % 8 != 0 || k % 8 != 0 || !fits(m, k) || !fits(m, n)) {  // the any-shape kernel
     const int64_t k_tiles = ceil_div(k, BM), col_tiles = ceil_div(n, ANY_BN);
     const int64_t blocks = static_cast<int64_t>(groups) * k_tiles * col_tiles;
-    BUX_CHECK(blocks < (1LL << 31), "bux_bf16_grouped_contract: too many tiles");
+    BUX_CHECK(blocks < (1LL << 31), "%s: too many tiles", name);
     hipLaunchKernelGGL(contract_any_kernel, dim3(static_cast<unsigned>(blocks)), dim3(THREADS), 0, s, x,
                        dy, groups, m, k, n, starts_in(workspace), k_tiles, col_tiles, dw);
     return launched("bf16 contract_any_kernel");
   }
   const int64_t d_tiles = ceil_div(k, BM), f_tiles = ceil_div(n, BN);
   const int64_t tiles = static_cast<int64_t>(groups) * d_tiles * f_tiles;
-  BUX_CHECK(tiles < (1LL << 31), "bux_bf16_grouped_contract: too many tiles");
+  BUX_CHECK(tiles < (1LL << 31), "%s: too many tiles", name);
   // K is the rows: A(r, i) = x[i][r] and B(c, i) = dy[i][c], both MN-major.
   const Operand A{x, static_cast<int32_t>(k), static_cast<int32_t>(m * k * 2), 0};
   const Operand B{dy, static_cast<int32_t>(n), static_cast<int32_t>(m * n * 2), 0};
@@ -887,38 +889,41 @@ static int contract_on(const uint16_t* x, const uint16_t* dy, const int32_t* siz
   return launched("bf16 contract_kernel");
 }
 
-extern "C" int bux_bf16_grouped_contract(const uint16_t* x, const uint16_t* dy, const int32_t* sizes,
-                                         int32_t groups, int64_t m, int64_t k, int64_t n,
-                                         uint16_t* dw, void* workspace, size_t workspace_bytes,
-                                         void* stream) {
-  using namespace bux;
-  clear_error();
-  BUX_CHECK(sizes != nullptr, "bux_bf16_grouped_contract: NULL buffer");
-  return contract_on(x, dy, sizes, groups, m, k, n, dw, workspace, workspace_bytes, stream);
-}
-
-extern "C" int bux_bf16_grouped_contract_listed(const uint16_t* x, const uint16_t* dy, int32_t groups, int64_t m, int64_t k, int64_t n,
-                                         uint16_t* dw, void* list, size_t list_bytes,
-                                         void* stream) {
-  bux::clear_error();
-  return contract_on(x, dy, nullptr, groups, m, k, n, dw, list, list_bytes, stream);
-}
-
-static int rows_f32_on(const float* x, const float* w, int w_transposed,
+extern "C" int bux_bf16_grouped_contract(const uint16_t* x, const uint16_t* dy,
                                          const int32_t* sizes, int32_t groups, int64_t m,
-                                         int64_t n, int64_t k, float* y, void* workspace,
+                                         int64_t k, int64_t n, uint16_t* dw, void* workspace,
                                          size_t workspace_bytes, void* stream) {
   using namespace bux;
-  BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS,
-            "bux_bf16_grouped_rows_f32: groups=%d outside [1, %d]", groups, MAX_GROUPS);
-  BUX_CHECK(m >= 0 && n > 0 && k > 0, "bux_bf16_grouped_rows_f32: bad shape m=%lld n=%lld k=%lld",
-            (long long)m, (long long)n, (long long)k);
-  BUX_CHECK(m < INT32_MAX, "bux_bf16_grouped_rows_f32: m=%lld rows", (long long)m);
-  BUX_CHECK(w && y && (m == 0 || x), "bux_bf16_grouped_rows_f32: NULL buffer");
+  const char* const name = "bux_bf16_grouped_contract";
+  clear_error();
+  BUX_CHECK(sizes != nullptr, "%s: NULL buffer", name);
+  return contract_on(name, x, dy, sizes, groups, m, k, n, dw, workspace, workspace_bytes, stream);
+}
+
+extern "C" int bux_bf16_grouped_contract_listed(const uint16_t* x, const uint16_t* dy,
+                                                int32_t groups, int64_t m, int64_t k, int64_t n,
+                                                uint16_t* dw, void* list, size_t list_bytes,
+                                                void* stream) {
+  using namespace bux;
+  const char* const name = "bux_bf16_grouped_contract_listed";
+  clear_error();
+  return contract_on(name, x, dy, nullptr, groups, m, k, n, dw, list, list_bytes, stream);
+}
+
+static int rows_f32_on(const char* name, const float* x, const float* w, int w_transposed,
+                       const int32_t* sizes, int32_t groups, int64_t m, int64_t n, int64_t k,
+                       float* y, void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace bux;
+  BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS, "%s: groups=%d outside [1, %d]", name, groups,
+            MAX_GROUPS);
+  BUX_CHECK(m >= 0 && n > 0 && k > 0, "%s: bad shape m=%lld n=%lld k=%lld", name, (long long)m,
+            (long long)n, (long long)k);
+  BUX_CHECK(m < INT32_MAX, "%s: m=%lld rows", name, (long long)m);
+  BUX_CHECK(w && y && (m == 0 || x), "%s: NULL buffer", name);
   const size_t need = bux_bf16_grouped_rows_workspace_size(groups, m);
   if (workspace == nullptr || workspace_bytes < need)
-    return fail(BUX_E_WORKSPACE, "bux_bf16_grouped_rows_f32: workspace of %zu bytes, %zu needed",
-                workspace_bytes, need);
+    return fail(BUX_E_WORKSPACE, "%s: %s of %zu bytes, %zu needed", name,
+                sizes ? "workspace" : "list", workspace_bytes, need);
   if (m == 0) return BUX_OK;
   hipStream_t s = as_stream(stream);
   if (sizes) {
@@ -929,7 +934,7 @@ static int rows_f32_on(const float* x, const float* w, int w_transposed,
   }
   const int64_t col_tiles = ceil_div(n, ANY_BN), slots = row_slots(groups, m, m);
   const int64_t blocks = slots * col_tiles;
-  BUX_CHECK(blocks < (1LL << 31), "bux_bf16_grouped_rows_f32: too many tiles");
+  BUX_CHECK(blocks < (1LL << 31), "%s: too many tiles", name);
   if (w_transposed)
     hipLaunchKernelGGL(rows_f32_kernel<true>, dim3(static_cast<unsigned>(blocks)), dim3(THREADS), 0,
                        s, x, w, groups, m, n, k, starts_in(workspace), tiles_in(workspace, groups),
@@ -946,36 +951,38 @@ extern "C" int bux_bf16_grouped_rows_f32(const float* x, const float* w, int w_t
                                          int64_t n, int64_t k, float* y, void* workspace,
                                          size_t workspace_bytes, void* stream) {
   using namespace bux;
+  const char* const name = "bux_bf16_grouped_rows_f32";
   clear_error();
-  BUX_CHECK(sizes != nullptr, "bux_bf16_grouped_rows_f32: NULL buffer");
-  return rows_f32_on(x, w, w_transposed, sizes, groups, m, n, k, y, workspace, workspace_bytes, stream);
+  BUX_CHECK(sizes != nullptr, "%s: NULL buffer", name);
+  return rows_f32_on(name, x, w, w_transposed, sizes, groups, m, n, k, y, workspace,
+                     workspace_bytes, stream);
 }
 
 extern "C" int bux_bf16_grouped_rows_listed_f32(const float* x, const float* w, int w_transposed,
-                                         int32_t groups, int64_t m,
-                                         int64_t n, int64_t k, float* y, void* list,
-                                         size_t list_bytes, void* stream) {
-  bux::clear_error();
-  return rows_f32_on(x, w, w_transposed, nullptr, groups, m, n, k, y, list, list_bytes, stream);
+                                                int32_t groups, int64_t m, int64_t n, int64_t k,
+                                                float* y, void* list, size_t list_bytes,
+                                                void* stream) {
+  using namespace bux;
+  const char* const name = "bux_bf16_grouped_rows_listed_f32";
+  clear_error();
+  return rows_f32_on(name, x, w, w_transposed, nullptr, groups, m, n, k, y, list, list_bytes,
+                     stream);
 }
 
-static int contract_f32_on(const float* x, const float* dy, const int32_t* sizes,
-                                             int32_t groups, int64_t m, int64_t k, int64_t n,
-                                             float* dw, void* workspace, size_t workspace_bytes,
-                                             void* stream) {
+static int contract_f32_on(const char* name, const float* x, const float* dy,
+                           const int32_t* sizes, int32_t groups, int64_t m, int64_t k, int64_t n,
+                           float* dw, void* workspace, size_t workspace_bytes, void* stream) {
   using namespace bux;
-  BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS,
-            "bux_bf16_grouped_contract_f32: groups=%d outside [1, %d]", groups, MAX_GROUPS);
-  BUX_CHECK(m >= 0 && n > 0 && k > 0,
-            "bux_bf16_grouped_contract_f32: bad shape m=%lld k=%lld n=%lld", (long long)m,
+  BUX_CHECK(groups >= 1 && groups <= MAX_GROUPS, "%s: groups=%d outside [1, %d]", name, groups,
+            MAX_GROUPS);
+  BUX_CHECK(m >= 0 && n > 0 && k > 0, "%s: bad shape m=%lld k=%lld n=%lld", name, (long long)m,
             (long long)k, (long long)n);
-  BUX_CHECK(m < INT32_MAX, "bux_bf16_grouped_contract_f32: m=%lld rows", (long long)m);
-  BUX_CHECK(dw && (m == 0 || (x && dy)), "bux_bf16_grouped_contract_f32: NULL buffer");
+  BUX_CHECK(m < INT32_MAX, "%s: m=%lld rows", name, (long long)m);
+  BUX_CHECK(dw && (m == 0 || (x && dy)), "%s: NULL buffer", name);
   const size_t need = bux_bf16_grouped_contract_workspace_size(groups);
   if (workspace == nullptr || workspace_bytes < need)
-    return fail(BUX_E_WORKSPACE,
-                "bux_bf16_grouped_contract_f32: workspace of %zu bytes, %zu needed",
-                workspace_bytes, need);
+    return fail(BUX_E_WORKSPACE, "%s: %s of %zu bytes, %zu needed", name,
+                sizes ? "workspace" : "list", workspace_bytes, need);
   hipStream_t s = as_stream(stream);
   if (sizes) {
     hipLaunchKernelGGL(prologue_kernel, dim3(1), dim3(THREADS), 0, s, sizes, groups, 0, 0, 1,
@@ -984,25 +991,30 @@ static int contract_f32_on(const float* x, const float* dy, const int32_t* sizes
   }
   const int64_t k_tiles = ceil_div(k, BM), col_tiles = ceil_div(n, ANY_BN);
   const int64_t blocks = static_cast<int64_t>(groups) * k_tiles * col_tiles;
-  BUX_CHECK(blocks < (1LL << 31), "bux_bf16_grouped_contract_f32: too many tiles");
+  BUX_CHECK(blocks < (1LL << 31), "%s: too many tiles", name);
   hipLaunchKernelGGL(contract_f32_kernel, dim3(static_cast<unsigned>(blocks)), dim3(THREADS), 0, s,
                      x, dy, groups, m, k, n, starts_in(workspace), k_tiles, col_tiles, dw);
   return launched("contract_f32_kernel");
 }
 
-extern "C" int bux_bf16_grouped_contract_f32(const float* x, const float* dy, const int32_t* sizes,
-                                             int32_t groups, int64_t m, int64_t k, int64_t n,
-                                             float* dw, void* workspace, size_t workspace_bytes,
-                                             void* stream) {
+extern "C" int bux_bf16_grouped_contract_f32(const float* x, const float* dy,
+                                             const int32_t* sizes, int32_t groups, int64_t m,
+                                             int64_t k, int64_t n, float* dw, void* workspace,
+                                             size_t workspace_bytes, void* stream) {
   using namespace bux;
+  const char* const name = "bux_bf16_grouped_contract_f32";
   clear_error();
-  BUX_CHECK(sizes != nullptr, "bux_bf16_grouped_contract_f32: NULL buffer");
-  return contract_f32_on(x, dy, sizes, groups, m, k, n, dw, workspace, workspace_bytes, stream);
+  BUX_CHECK(sizes != nullptr, "%s: NULL buffer", name);
+  return contract_f32_on(name, x, dy, sizes, groups, m, k, n, dw, workspace, workspace_bytes,
+                         stream);
 }
 
-extern "C" int bux_bf16_grouped_contract_listed_f32(const float* x, const float* dy, int32_t groups, int64_t m, int64_t k, int64_t n,
-                                             float* dw, void* list, size_t list_bytes,
-                                             void* stream) {
-  bux::clear_error();
-  return contract_f32_on(x, dy, nullptr, groups, m, k, n, dw, list, list_bytes, stream);
+extern "C" int bux_bf16_grouped_contract_listed_f32(const float* x, const float* dy,
+                                                    int32_t groups, int64_t m, int64_t k,
+                                                    int64_t n, float* dw, void* list,
+                                                    size_t list_bytes, void* stream) {
+  using namespace bux;
+  const char* const name = "bux_bf16_grouped_contract_listed_f32";
+  clear_error();
+  return contract_f32_on(name, x, dy, nullptr, groups, m, k, n, dw, list, list_bytes, stream);
 }

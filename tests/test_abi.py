@@ -386,3 +386,38 @@ def test_the_norm_backwards_workspace_never_falls_as_rows_grow(lib):
                  for m in [*range(0, 4200), *range(65000, 66700), 131072, 1 << 20]]
         assert sizes == sorted(sizes)
         assert sizes[0] == 0 and sizes[1] == 8 * d
+
+
+@pytest.mark.parametrize("twin", ["", "_f32"])
+def test_listed_compute_gemms_reject_bad_arguments(lib, twin):
+    """Each listed GEMM checks its list as its unlisted form checks its workspace, and
+    names itself and the list in the error."""
+    p = ctypes.c_void_p(16)
+    rows, contract = (f"bux_bf16_grouped_{kind}_listed{twin}" for kind in ("rows", "contract"))
+    need = lib.bux_bf16_grouped_rows_workspace_size(4, 64)
+    cases = [(rows, (p, p, 0, 4, 64, 100, 37, p, None, need, None), 2, "list of"),
+             (rows, (p, p, 0, 4, 64, 100, 37, p, p, need - 1, None), 2, f"list of {need - 1} bytes"),
+             (rows, (p, p, 0, 0, 64, 100, 37, p, p, need, None), 1, "groups=0"),
+             (rows, (p, None, 0, 4, 64, 100, 37, p, p, need, None), 1, "NULL"),
+             (contract, (p, p, 4, 64, 45, 100, p, None, 1 << 10, None), 2, "list of"),
+             (contract, (p, p, 4, 64, 45, 100, p, p, 8, None), 2, "list of 8 bytes"),
+             (contract, (p, p, 4, 64, 0, 100, p, p, 1 << 10, None), 1, "k=0")]
+    for name, args, code, text in cases:
+        rc = getattr(lib, name)(*args)
+        assert rc == code and text in _msg(lib) and name + ":" in _msg(lib), (name, rc, _msg(lib))
+
+
+def test_biased_rows_reject_bad_arguments(lib):
+    p = ctypes.c_void_p(16)
+    need = lib.bux_mx_grouped_rows_workspace_size(4, 256, 200)
+
+    def rows(values=p, list_at=p, list_bytes=need, groups=4, k=128, bias=p):
+        return lib.bux_mx_grouped_rows_biased(values, p, p, p, list_at, list_bytes, groups, 256, 128, k,
+                                              200, 0, bias, p, None)
+
+    assert rows(list_at=None) == 1 and "NULL list or bias" in _msg(lib)
+    assert rows(bias=None) == 1 and "NULL list or bias" in _msg(lib)
+    assert rows(list_bytes=need - 1) == 2 and "groups=4" in _msg(lib)
+    assert rows(k=100) == 1 and "k=100" in _msg(lib)
+    assert rows(values=None) == 1 and "NULL buffer" in _msg(lib)
+    assert "bux_mx_grouped_rows_biased" in _msg(lib)

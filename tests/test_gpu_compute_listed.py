@@ -57,3 +57,29 @@ def test_a_contract_on_a_list_of_more_rows(lib, kind):
     torch.cuda.synchronize()
     assert torch.equal(own, listed)
     assert bool((own[:1] != 0).any()) and not own[4].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("k,n", [(64, 264), (45, 37)])
+def test_a_list_of_other_dimensions_is_refused_by_the_kernel(lib, k, n, dtype):
+    """Through the C ABI, which sees a list's size alone: the GEMM writes nothing and sets
+    the list's status word."""
+    from bux_amd import grouped_mxfp8, kernels
+    m, groups = 200, 3
+    gs = torch.tensor([100, 40, 60], dtype=torch.int32, device="cuda")
+    x, w, dy, y, dw = (torch.full(s, 3.0, device="cuda", dtype=dtype)
+                       for s in ((m, k), (groups, k, n), (m, n), (m, n), (groups, k, n)))
+    twin = "_f32" if dtype == torch.float32 else ""
+    p, s = kernels.ptr, kernels.stream()
+    announce("lists of other dimensions", k, n, dtype)
+    lists = {"rows": (gs, m + 56, m), "contract": (torch.cat([gs, gs]), m, m)}
+    for kind, args in lists.items():
+        made = grouped_mxfp8.tiles_of(*args)
+        call = getattr(lib, f"bux_bf16_grouped_{kind}_listed{twin}")
+        size = made.buffer.numel()
+        rc = (call(p(x), p(w), 0, groups, m, n, k, p(y), p(made.buffer), size, s) if kind == "rows"
+              else call(p(x), p(dy), groups, m, k, n, p(dw), p(made.buffer), size, s))
+        torch.cuda.synchronize()
+        status = made.buffer[:20].view(torch.int32)[4].item()
+        assert rc == 0 and status == 1  # BUX_LIST_REFUSED
+    assert bool((y == 3).all()) and bool((dw == 3).all())
