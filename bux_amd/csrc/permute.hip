@@ -263,10 +263,11 @@ constexpr int64_t SMALL_PICKS = 8192;
 constexpr int SMALL_BINS = 900;  // at most SMALL_THREADS: a thread a bin
 
 // Its LDS: the waves' counts, the offsets, the order, the sorted weights (16-byte aligned).
-__host__ __device__ __forceinline__ size_t small_lds(int32_t n, int32_t bins, int32_t word) {
+__host__ __device__ constexpr size_t small_lds(int32_t n, int32_t bins, int32_t word) {
   const size_t ints = (static_cast<size_t>(SMALL_WAVES + 1) * bins + n + 3) / 4 * 4;
   return ints * sizeof(int32_t) + static_cast<size_t>(n) * word;
 }
+static_assert(small_lds(SMALL_PICKS, SMALL_BINS, 4) <= 152 * 1024, "small_kernel fits a CU's LDS");
 
 template <int TURNS>
 __global__ __launch_bounds__(SMALL_THREADS) void small_kernel(
@@ -367,11 +368,9 @@ int permute(const char* name, const int32_t* idx, int64_t n_picks, int32_t num_e
   int bits = 0;
   while ((1 << bits) < bins) ++bits;
   hipStream_t s = as_stream(stream);
-  const size_t small = n_picks <= SMALL_PICKS
-                           ? small_lds(static_cast<int32_t>(n_picks), bins, outs.row_weights ? outs.word : 0)
-                           : 0;
-  if (n_picks <= SMALL_PICKS && bins <= SMALL_BINS && small <= 152 * 1024) {
-    const size_t lds = small;
+  if (n_picks <= SMALL_PICKS && bins <= SMALL_BINS) {
+    const size_t lds =
+        small_lds(static_cast<int32_t>(n_picks), bins, outs.row_weights ? outs.word : 0);
     auto go = [&](auto kernel) {
       if (lds > 64 * 1024)
         if (int rc = allow_lds(kernel, lds, "small_kernel")) return rc;
