@@ -196,9 +196,12 @@ __global__ __launch_bounds__(SCAN_THREADS) void bases_kernel(const int32_t* __re
   }
 }
 
-// The places of a wave's next 64 picks, in order: lane l's pick in bin b (`valid`: it has
-// one); `running` (LDS, the wave's own): where each bin's next pick goes.
-__device__ __forceinline__ int32_t place(int b, bool valid, int32_t bits, int32_t* running) {
+// A wave's next 64 picks, lane l's in bin b (`valid`: it has one): how many of them share
+// the lane's bin, and how many of those come before it.
+struct Peers {
+  int32_t count, rank;
+};
+__device__ __forceinline__ Peers peers_of(int b, bool valid, int32_t bits) {
   const uint64_t below = (1ull << (threadIdx.x & 63)) - 1ull;
   uint64_t peers = __ballot(valid);
   for (int bit = 0; bit < bits; ++bit) {
@@ -206,12 +209,17 @@ __device__ __forceinline__ int32_t place(int b, bool valid, int32_t bits, int32_
     const uint64_t m = __ballot(set);
     peers &= set ? m : ~m;
   }
-  const int rank = __popcll(peers & below);
+  return Peers{static_cast<int32_t>(__popcll(peers)), static_cast<int32_t>(__popcll(peers & below))};
+}
+
+// The picks' places, in order; `running` (LDS, the wave's own): where each bin's next pick
+// goes.
+__device__ __forceinline__ int32_t place(int b, bool valid, const Peers& peers, int32_t* running) {
   const int32_t start = valid ? running[b] : 0;
   __builtin_amdgcn_wave_barrier();
-  if (valid && rank == 0) running[b] = start + __popcll(peers);
+  if (valid && peers.rank == 0) running[b] = start + peers.count;
   __builtin_amdgcn_wave_barrier();
-  return start + rank;
+  return start + peers.rank;
 }
 
 __global__ __launch_bounds__(64 * WAVES) void scatter_kernel(
@@ -241,7 +249,7 @@ __global__ __launch_bounds__(64 * WAVES) void scatter_kernel(
 #pragma unroll
   for (int i = 0; i < TURNS; ++i) {
     const int64_t p = p0 + 64 * i;
-    const int32_t pos = place(bin[i], p < n, bits, running);
+    const int32_t pos = place(bin[i], p < n, peers_of(bin[i], p < n, bits), running);
     if (p >= n) continue;
     order[pos] = static_cast<int32_t>(p);
     inverse[p] = pos;
@@ -252,7 +260,7 @@ __global__ __launch_bounds__(64 * WAVES) void scatter_kernel(
 // The whole sort by one workgroup: wave w takes the picks [w per, (w + 1) per). A wave's
 // picks and weights are read at once (TURNS of 64), and the order and the sorted weights
 // are put together in LDS and written in runs (scattered from one CU, a store of 64 lines
-// holds its memory pipe 64 cycles). What bounds it is one CU's VALU: `place` takes 16
+// holds its memory pipe 64 cycles). What bounds it is one CU's VALU: `peers_of` takes 16
 // waves' 1024 picks in about 1 us. In a graph, with weights and list, against the four
 // kernels and the two the layer ran after them (us): 64 picks 4.8 and 21, 1600 picks 5.9
 // and 20. Alone 8192 picks take 9.4, 16000 would take 19; the four kernels take 12 to 13
@@ -294,9 +302,16 @@ __global__ __launch_bounds__(SMALL_THREADS) void small_kernel(
   }
   for (int b = lane; b < bins; b += 64) mine[b] = 0;
   __builtin_amdgcn_wave_barrier();
+  // one lane adds a bin's picks of a turn: a lane a pick, 8192 picks all in one bin took 15.5
+  // us (the additions to one address go one after another), now 9.4
+  Peers peers[TURNS];
 #pragma unroll
-  for (int i = 0; i < TURNS; ++i)
-    if (p0 + 64 * i < end) atomicAdd(&mine[bin[i]], 1);
+  for (int i = 0; i < TURNS; ++i) {
+    if (p0 - lane + 64 * i >= end) break;  // the whole wave
+    const bool valid = p0 + 64 * i < end;
+    peers[i] = peers_of(bin[i], valid, bits);
+    if (valid && peers[i].rank == 0) atomicAdd(&mine[bin[i]], peers[i].count);
+  }
   __syncthreads();
   const int b = threadIdx.x;
   int32_t total = 0;
@@ -321,7 +336,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void small_kernel(
   for (int i = 0; i < TURNS; ++i) {
     const int32_t p = p0 + 64 * i;
     if (p - lane >= end) break;  // the whole wave
-    const int32_t pos = place(bin[i], p < end, bits, mine);
+    const int32_t pos = place(bin[i], p < end, peers[i], mine);
     if (p >= end) continue;
     sorted[pos] = p;
     inverse[p] = pos;

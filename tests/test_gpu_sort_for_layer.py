@@ -61,3 +61,20 @@ def test_weights_other_than_one_a_pick(lib):
     torch.cuda.synchronize()
     assert strided.tolist() == [4, 2, 1, 5, 3, 6]  # order 1, 2, 0, 3, 4, 5 of 1 4 2 5 3 6
     assert short.tolist() == [2, 3, 1, 4, 0, 0]
+
+
+@pytest.mark.parametrize("n", [64, 1000, 4097, 8192])
+def test_picks_of_few_experts(lib, n):
+    """All the picks with one expert, and in runs of two: a wave's 64 picks in a bin or two,
+    in the one-workgroup kernel with one to eight turns a wave and a last one in part."""
+    from bux_amd import moe
+    announce("layer sort, picks of few experts", n)
+    for idx in (np.full((n, 1), 5, np.int32), (np.arange(n, dtype=np.int32)[:, None] // 37) % 2 + 3):
+        weights = torch.randn(n, 1, device="cuda")
+        s, row_weights, _ = moe.sort_for_layer(to_gpu(idx), 8, weights, None)
+        torch.cuda.synchronize()
+        want = omoe.sort_by_expert(idx, 8)
+        np.testing.assert_array_equal(s.order.cpu().numpy(), want.order)
+        np.testing.assert_array_equal(s.inverse.cpu().numpy(), want.inverse)
+        np.testing.assert_array_equal(s.sizes.cpu().numpy(), want.sizes)
+        assert torch.equal(row_weights, weights.reshape(-1)[s.order.long()])
