@@ -385,8 +385,8 @@ __device__ __forceinline__ void stream8(void* at, uint32_t x, uint32_t y) {
 // float32 through the wave's region of the stage, 32 rows x 64 columns (a row's 256 bytes,
 // rows 272 apart) at a time: read back 16 bytes a lane, 16 lanes a row, a store writes
 // 4 whole rows of 256 bytes. (Straight from the accumulators a store instruction wrote
-// 32 rows of 32 bytes: config 3's up wgrad into float32, 1.6 GB of outputs, took 1494 us,
-// this way 627.) I, J: the wave's blocks of 32 rows and columns, its first row and column
+// 32 rows of 32 bytes: config 3's up wgrad into float32, 1.6 GB of outputs, took 1528 us,
+// this way 575.) I, J: the wave's blocks of 32 rows and columns, its first row and column
 // row0 and col0 of the tile; the rows [0, rows) and columns [0, cols) are stored (cols a
 // multiple of 4).
 template <int I, int J, typename Values>
@@ -398,6 +398,14 @@ __device__ void store_f32(const Values& values, float* tile, int32_t ld, int32_t
   uint8_t* mine = region + (lane & 31) * FP + 16 * (lane >> 5);
   const int cc = lane & 15;
   const uint8_t* from = region + (lane >> 4) * FP + cc * 16;
+  // a lane's first output, its others a scalar offset away: an address a row took 90
+  // registers, which went to scratch memory (the contract above 609 us with them)
+  float* const out = tile + (row0 + (lane >> 4)) * ld + col0 + 4 * cc;
+  float4 bias[J / 2];
+  if constexpr (Values::BIASED) {
+#pragma unroll
+    for (int jj = 0; jj < J; jj += 2) bias[jj / 2] = values.bias4(col0 + jj * 32 + 4 * cc, cols);
+  }
 #pragma unroll
   for (int i = 0; i < I; ++i)
 #pragma unroll
@@ -412,12 +420,21 @@ __device__ void store_f32(const Values& values, float* tile, int32_t ld, int32_t
       uint4 v[8];
 #pragma unroll
       for (int it = 0; it < 8; ++it) v[it] = *reinterpret_cast<const uint4*>(from + it * 4 * FP);
+      if constexpr (Values::BIASED) {
+        const float4& b = bias[jj / 2];
+#pragma unroll
+        for (int it = 0; it < 8; ++it)
+          v[it] = make_uint4(__float_as_uint(__uint_as_float(v[it].x) + b.x),
+                             __float_as_uint(__uint_as_float(v[it].y) + b.y),
+                             __float_as_uint(__uint_as_float(v[it].z) + b.z),
+                             __float_as_uint(__uint_as_float(v[it].w) + b.w));
+      }
       const int32_t col = col0 + jj * 32 + 4 * cc;
       if (col < cols) {
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
           const int32_t row = row0 + i * 32 + it * 4 + (lane >> 4);
-          if (row < rows) stream16(tile + row * ld + col, v[it]);
+          if (row < rows) stream16(out + (i * 32 + it * 4) * ld + jj * 32, v[it]);
         }
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -443,6 +460,7 @@ __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
 }
 struct FromAcc {
+  static constexpr bool BIASED = false;
   const v16f (*acc)[4];
   __device__ __forceinline__ uint2 operator()(int i, int j, int g) const {
     const v16f& a = acc[i][j];
@@ -456,7 +474,9 @@ struct FromAcc {
 
 // FromAcc's values with their column's bias added as an op of its own does: the product
 // rounded to the output's type, then the sum. A tile holds one group's rows, so a lane's
-// biases are those of its columns, 4 a run: read once a tile, before the stores.
+// biases are those of its columns, read once a tile, before the stores: 4 a run of the
+// accumulators in bfloat16; in float32 those of the columns that the lane reads back from
+// LDS (all of its runs' would take 64 registers, and spilled).
 struct FromAccBiased16 {
   FromAcc from;
   uint2 bias[4][4];
@@ -469,12 +489,12 @@ struct FromAccBiased16 {
     return make_uint2(add(v.x, bias[j][g].x), add(v.y, bias[j][g].y));
   }
 };
-struct FromAccBiased32 {
-  FromAcc from;
-  float4 bias[4][4];
-  __device__ __forceinline__ float4 f32(int i, int j, int g) const {
-    const float4 v = from.f32(i, j, g), b = bias[j][g];
-    return make_float4(v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w);
+struct FromAccBiased32 : FromAcc {
+  static constexpr bool BIASED = true;
+  const float* row;  // the group's biases from the tile's first column on; NULL for none
+  __device__ __forceinline__ float4 bias4(int32_t col, int32_t cols) const {
+    return row != nullptr && col < cols ? *reinterpret_cast<const float4*>(row + col)
+                                        : make_float4(0, 0, 0, 0);
   }
 };
 
@@ -683,8 +703,7 @@ struct Plain {
 
 // A lane's biases of its columns, from the group's row at the tile's first column: run g of
 // block b takes columns 8 g + 4 (l / 32) .. + 3 of those 32 (`first` the wave's first).
-template <typename Run, typename T>
-__device__ __forceinline__ void read_bias(Run (&bias)[4][4], const T* row, int32_t first,
+__device__ __forceinline__ void read_bias(uint2 (&bias)[4][4], const uint16_t* row, int32_t first,
                                           int32_t cols, int32_t blocks) {
   first += 4 * ((threadIdx.x & 63) >> 5);
 #pragma unroll
@@ -692,7 +711,7 @@ __device__ __forceinline__ void read_bias(Run (&bias)[4][4], const T* row, int32
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int32_t col = first + b * 32 + 8 * g;  // columns are a multiple of 4
-      bias[b][g] = b < blocks && col < cols ? *reinterpret_cast<const Run*>(row + col) : Run{};
+      bias[b][g] = b < blocks && col < cols ? *reinterpret_cast<const uint2*>(row + col) : uint2{};
     }
 }
 
@@ -707,13 +726,16 @@ struct PlainBiased {
   int32_t ld;
   const T* bias;
   __device__ __forceinline__ void store(const v16f acc[4][4], const Job& j, Stage& stage) const {
-    const int wave = threadIdx.x >> 6;
     const T* row = bias + static_cast<int64_t>(j.group) * ld + j.b_row0;
-    const int32_t first = j.half ? wave * 64 : (wave & 1) * 128;  // the wave's columns
-    std::conditional_t<std::is_same<T, uint16_t>::value, FromAccBiased16, FromAccBiased32> from{
-        FromAcc{acc}};
-    read_bias(from.bias, row, first, j.n > 0 ? j.cols : 0, j.half ? 2 : 4);
-    store_plain(from, out, ld, j, stage);
+    if constexpr (std::is_same<T, uint16_t>::value) {
+      const int wave = threadIdx.x >> 6;
+      const int32_t first = j.half ? wave * 64 : (wave & 1) * 128;  // the wave's columns
+      FromAccBiased16 from{FromAcc{acc}};
+      read_bias(from.bias, row, first, j.n > 0 ? j.cols : 0, j.half ? 2 : 4);
+      store_plain(from, out, ld, j, stage);
+    } else {
+      store_plain(FromAccBiased32{{acc}, j.n > 0 ? row : nullptr}, out, ld, j, stage);
+    }
   }
 };
 
