@@ -25,7 +25,7 @@
 //
 // Both are bound by a row's chain of loads and block sums (about 4 us a row backward), so
 // what counts is the rows in flight: the chunks are a template parameter, which keeps the
-// registers of a narrow row (d 1024: 188 -> 60) from holding four workgroups' worth of a
+// registers of a narrow row (backward, d 1024: 256 -> 122) from holding four workgroups' worth of a
 // CU, and a backward workgroup takes few rows where there are few (64 each put 4004 rows
 // on 63 CUs: 259 us in float32 at d 1024, and 19 us for the partials; now 25 and 9).
 
@@ -42,12 +42,22 @@ constexpr int VEC = 8;
 constexpr int MAX_CHUNKS = 4;  // d <= MAX_CHUNKS * THREADS * VEC = 8192
 constexpr int MAX_ROWS = 64;   // rows a backward workgroup, at most
 
-// The backward's workgroups over m rows: a row each up to 1024 (4 a CU), then 1024 until
-// they take MAX_ROWS each. It never falls as m grows: a workspace for the most rows a caller
-// has serves fewer too.
-int64_t backward_blocks(int64_t m) {
-  const int64_t most = m < 1024 ? m : 1024, least = ceil_div(m, MAX_ROWS);
-  return most > least ? most : least;
+// Calls f(std::integral_constant<int, C>{}) for a row of d columns in C chunks.
+template <typename F>
+auto with_chunks(int64_t d, F&& f) {
+  if (d <= THREADS * VEC) return f(std::integral_constant<int, 1>{});
+  if (d <= 2 * THREADS * VEC) return f(std::integral_constant<int, 2>{});
+  return f(std::integral_constant<int, MAX_CHUNKS>{});
+}
+
+// The backward's workgroups over m rows of C chunks: a row each up to as many as the chip
+// holds at once by their registers (4, 2 or 1 a CU), then that many, and past MAX_ROWS rows
+// each a multiple of it. It never falls as m grows, so that a workspace for the most rows a
+// caller has serves fewer too. (Float32: 1024 rows of 7168 on 1024 workgroups took 87 us, on
+// 256 they take 50; 40000 rows of 7168 on 625 workgroups 1812, on 768 1515.)
+int64_t backward_blocks(int64_t m, int chunks) {
+  const int64_t at_once = 1024 / chunks;
+  return m < at_once ? m : ceil_div(m, at_once * MAX_ROWS) * at_once;
 }
 
 // The sum of v over the workgroup (256 threads); `red` 4 floats of LDS. Every thread
@@ -325,14 +335,6 @@ __global__ __launch_bounds__(PARAM_THREADS) void norm_params_kernel(
   if (out) out[c] = sum;
 }
 
-// Calls f(std::integral_constant<int, C>{}) for a row of d columns in C chunks.
-template <typename F>
-void with_chunks(int64_t d, F&& f) {
-  if (d <= THREADS * VEC) f(std::integral_constant<int, 1>{});
-  else if (d <= 2 * THREADS * VEC) f(std::integral_constant<int, 2>{});
-  else f(std::integral_constant<int, MAX_CHUNKS>{});
-}
-
 template <typename T>
 int norm_args(const char* name, const bux_norm* norm, const T* scale, const T* bias,
               const T* down_bias, const int32_t* offsets, int32_t experts, NormArgs<T>* a) {
@@ -373,8 +375,17 @@ int norm_forward(const char* name, const T* y, int64_t m, int64_t d, const T* do
   return launched("norm_forward_kernel");
 }
 
+// Two sums a workgroup and column. Wider rows have fewer workgroups: the most that any
+// narrower row takes, so that it does not fall as d grows either.
 size_t backward_workspace(int64_t m, int64_t d) {
-  return static_cast<size_t>(2 * backward_blocks(m) * d) * sizeof(float);
+  int64_t columns = 0;
+  for (int chunks = 1; chunks <= MAX_CHUNKS; chunks *= 2) {
+    const int64_t widest = static_cast<int64_t>(chunks) * THREADS * VEC;
+    const int64_t c = backward_blocks(m, chunks) * (d < widest ? d : widest);
+    columns = c > columns ? c : columns;
+    if (d <= widest) break;
+  }
+  return static_cast<size_t>(2 * columns) * sizeof(float);
 }
 
 template <typename T>
@@ -395,7 +406,7 @@ int norm_backward(const char* name, const T* dy, const int32_t* index, int32_t i
     return fail(BUX_E_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", name, workspace_bytes,
                 need);
   hipStream_t s = as_stream(stream);
-  const int64_t blocks = backward_blocks(m);
+  const int64_t blocks = with_chunks(d, [&](auto c) { return backward_blocks(m, decltype(c)::value); });
   if (m > 0) {
     BUX_CHECK(dy && y && weights && dv && d_weights, "%s: NULL buffer", name);
     with_chunks(d, [&](auto c) {

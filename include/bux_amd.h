@@ -461,9 +461,9 @@ int bux_expert_bias_weight_grad_f32(const float* dy, const int32_t* index, int32
  * expert, to the down bias: bux_expert_sums of it); d_weights [m] (written: the norm
  * path's only use of the weights); d_scale and d_bias [d] float32 sums over the rows
  * (NULL where the norm has none). workspace:
- * bux_expert_norm_backward_workspace_size(m, d) bytes: 8 d for each of min(m, 1024)
- * workgroups (ceil(m / 64) past 65536 rows). It never falls as m grows, so that one of a
- * caller's largest m serves every smaller one.
+ * bux_expert_norm_backward_workspace_size(m, d) bytes, at most 8 m d and at most 16 MiB +
+ * m d / 8. It never falls as m or d grows, so that one of a caller's largest serves every
+ * smaller one.
  */
 enum { BUX_LAYERNORM = 0, BUX_RMSNORM = 1 };
 typedef struct bux_norm {

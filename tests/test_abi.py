@@ -379,13 +379,19 @@ def test_the_layers_sort_rejects_bad_arguments(lib):
 
 
 def test_the_norm_backwards_workspace_never_falls_as_rows_grow(lib):
-    """One sized for a caller's largest m serves every smaller one, around the rows at
-    which its workgroups take one more row each and at which they take their most."""
-    for d in (8, 2056, 7168):
-        sizes = [lib.bux_expert_norm_backward_workspace_size(m, d)
-                 for m in [*range(0, 4200), *range(65000, 66700), 131072, 1 << 20]]
+    """One sized for a caller's largest m and d serves every smaller one, around the rows
+    at which its workgroups take one more row each and at which they take their most, and
+    the columns at which a row takes another chunk."""
+    size = lib.bux_expert_norm_backward_workspace_size
+    for d in (8, 2048, 2056, 4096, 7168):
+        sizes = [size(m, d) for m in [*range(0, 4200), *range(16300, 16500), *range(65000, 66700),
+                                      131072, 1 << 20]]
         assert sizes == sorted(sizes)
         assert sizes[0] == 0 and sizes[1] == 8 * d
+        assert size(1 << 20, d) <= (16 << 20) + (1 << 20) * d // 8
+    for m in (1, 255, 257, 511, 1000, 1025, 16385, 70000):
+        sizes = [size(m, d) for d in range(8, 8200, 8)]
+        assert sizes == sorted(sizes)
 
 
 @pytest.mark.parametrize("twin", ["", "_f32"])
