@@ -86,6 +86,16 @@ struct NormArgs {
   int32_t experts;
 };
 
+// The chunks a loop over a row of d columns takes: C, or in bfloat16 with C the most, those
+// that d has. (Leaving those loops early keeps the forward at 84 registers; without, it takes
+// 102, a wave a SIMD less: 65536 rows of 7168 took 789 us, now 670. Float32 takes 108 either
+// way, and 64 rows of 7168 go 5.8 -> 5.5 us without.)
+template <typename T, int C>
+__device__ __forceinline__ int chunks_of(int64_t d) {
+  return std::is_same<T, uint16_t>::value && C == MAX_CHUNKS
+             ? static_cast<int>((d + THREADS * VEC - 1) / (THREADS * VEC)) : C;
+}
+
 // One thread's share of a row of C chunks: columns c(i) = (i * THREADS + threadIdx.x) * VEC + j.
 template <int C>
 struct Row {
@@ -139,6 +149,7 @@ __device__ __forceinline__ void norm_stats(const NormArgs<T>& a, const Row<C>& x
   float q = 0.0f;
 #pragma unroll
   for (int i = 0; i < C; ++i) {
+    if (i >= chunks_of<T, C>(d)) break;
     const int64_t c = (static_cast<int64_t>(i) * THREADS + threadIdx.x) * VEC;
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
@@ -177,6 +188,7 @@ __global__ __launch_bounds__(THREADS) void norm_forward_kernel(
   const float w = E::value(weights[r]);
 #pragma unroll
   for (int i = 0; i < C; ++i) {
+    if (i >= chunks_of<T, C>(d)) break;
     const int64_t c = (static_cast<int64_t>(i) * THREADS + threadIdx.x) * VEC;
     if (c >= d) continue;
     float b[VEC] = {0, 0, 0, 0, 0, 0, 0, 0}, v[VEC];
