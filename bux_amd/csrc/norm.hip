@@ -18,16 +18,17 @@
 // groups: the picks outside the experts, whose weights the layer zeroes) give 0.
 //
 // Forward: a workgroup a row, the row in registers (d <= 8192: 8 values a thread a 2048
-// chunk), block sums through LDS. Backward: a workgroup of backward_blocks takes an even share
-// of the rows one after another, each thread the same columns of every row, so that it adds its columns' gain and
-// bias gradients over the rows in registers; one float32 partial a workgroup and column
-// goes to the workspace, and norm_params_kernel adds the partials in a fixed order.
+// chunk), block sums through LDS. Backward: a workgroup of backward_blocks takes an even
+// share of the rows one after another, each thread the same columns of every row, so that it
+// adds its columns' gain and bias gradients over the rows in registers; one float32 partial a
+// workgroup and column goes to the workspace, and norm_params_kernel adds the partials in a
+// fixed order.
 //
 // Both are bound by a row's chain of loads and block sums (about 4 us a row backward), so
 // what counts is the rows in flight: the chunks are a template parameter, which keeps the
-// registers of a narrow row (backward, d 1024: 256 -> 122) from holding four workgroups' worth of a
-// CU, and a backward workgroup takes few rows where there are few (64 each put 4004 rows
-// on 63 CUs: 259 us in float32 at d 1024, and 19 us for the partials; now 25 and 9).
+// registers of a narrow row few (backward, d 1024: 256 -> 122, four workgroups a CU), and a
+// backward workgroup takes few rows where there are few (64 each put 4004 rows on 63 CUs:
+// 259 us in float32 at d 1024, and 19 us for the partials; now 25 and 9).
 
 #include <type_traits>
 

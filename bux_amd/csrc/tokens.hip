@@ -450,35 +450,33 @@ __global__ __launch_bounds__(THREADS) void expert_bias_add_kernel(
 }
 
 // out[e] = sum over e's rows of v_r (x[src(r)], times weights[r] rounded to T if
-// weights). Workgroup (e, 256 columns): its 16 waves add every 16th row of e in order, four
-// rows' loads in flight and lanes 4 columns each; the waves' sums are added in wave order.
-// Deterministic. What bounds it is the rows a wave adds one after another: 16 experts of
-// 250 rows of 1024 float32 took 28 us by 4 waves of 512 columns (32 workgroups), now 6.5.
-constexpr int SUM_THREADS = 1024;
-constexpr int SUM_VEC = 4;
-constexpr int SUM_COLS = 64 * SUM_VEC;  // a workgroup's columns
-template <typename T>
-__global__ __launch_bounds__(SUM_THREADS) void expert_sums_kernel(
+// weights). Workgroup (e, 64 N columns): its WAVES waves add every WAVES-th row of e in
+// order, AT_ONCE rows' loads in flight and lanes N columns each; the waves' sums are added
+// in wave order. Deterministic. Which form a call takes: expert_sums.
+template <typename T, int WAVES, int N, int AT_ONCE>
+__global__ __launch_bounds__(WAVES * 64) void expert_sums_kernel(
     const T* __restrict__ x, const int32_t* __restrict__ index, int32_t index_div,
     int64_t sources, const T* __restrict__ weights, int64_t m, int64_t width,
     const int32_t* __restrict__ offsets, int32_t experts, float* __restrict__ out) {
   // Each product rounds before it is added, as the reference's ops do (no FMA contraction).
 #pragma clang fp contract(off)
   using E = Elem<T>;
-  constexpr int WAVES = SUM_THREADS / 64, AT_ONCE = 4;
-  __shared__ float part[WAVES][SUM_COLS];
-  const int64_t chunks = (width + SUM_COLS - 1) / SUM_COLS;
+  constexpr int COLS = 64 * N;
+  __shared__ float part[WAVES][COLS];
+  const int64_t chunks = (width + COLS - 1) / COLS;
   const int64_t e = blockIdx.x / chunks;
-  const int64_t c0 = (blockIdx.x % chunks) * SUM_COLS;
+  const int64_t c0 = (blockIdx.x % chunks) * COLS;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t c = c0 + lane * SUM_VEC;
+  const int64_t c = c0 + lane * N;
   // rows inside [0, m) only, whatever the offsets say
   const int64_t lo = offsets[e] > 0 ? offsets[e] : 0;
   const int64_t hi = offsets[e + 1] < m ? offsets[e + 1] : m;
-  float acc[SUM_VEC] = {0, 0, 0, 0};
+  float acc[N];
+#pragma unroll
+  for (int q = 0; q < N; ++q) acc[q] = 0.0f;
   if (c < width) {  // width is a multiple of 8: a lane's columns are all in or out
     for (int64_t r0 = lo + wave; r0 < hi; r0 += WAVES * AT_ONCE) {
-      float v[AT_ONCE][SUM_VEC];
+      float v[AT_ONCE][N];
       bool live[AT_ONCE];
 #pragma unroll
       for (int i = 0; i < AT_ONCE; ++i) {
@@ -486,28 +484,29 @@ __global__ __launch_bounds__(SUM_THREADS) void expert_sums_kernel(
         const int64_t src = r >= hi ? -1 : (index ? source_row(index[r], index_div, sources) : r);
         live[i] = src >= 0;  // else past the rows, or a row of 0
         if (!live[i]) continue;
-        load4(x + src * width + c, v[i]);
+        if constexpr (N == 8) E::load8(x + src * width + c, v[i]);
+        else load4(x + src * width + c, v[i]);
         if (weights) {
           const float w = E::value(weights[r]);
 #pragma unroll
-          for (int q = 0; q < SUM_VEC; ++q) v[i][q] = E::round(v[i][q] * w);
+          for (int q = 0; q < N; ++q) v[i][q] = E::round(v[i][q] * w);
         }
       }
 #pragma unroll
       for (int i = 0; i < AT_ONCE; ++i)
 #pragma unroll
-        for (int q = 0; q < SUM_VEC; ++q) acc[q] = live[i] ? acc[q] + v[i][q] : acc[q];
+        for (int q = 0; q < N; ++q) acc[q] = live[i] ? acc[q] + v[i][q] : acc[q];
     }
   }
 #pragma unroll
-  for (int q = 0; q < SUM_VEC; ++q) part[wave][lane * SUM_VEC + q] = acc[q];
+  for (int q = 0; q < N; ++q) part[wave][lane * N + q] = acc[q];
   __syncthreads();
-  const int j = threadIdx.x;  // a thread a column
-  if (j >= SUM_COLS || c0 + j >= width) return;
-  float sum = part[0][j];
+  for (int j = threadIdx.x; j < COLS && c0 + j < width; j += WAVES * 64) {  // a thread a column
+    float sum = part[0][j];
 #pragma unroll
-  for (int w = 1; w < WAVES; ++w) sum += part[w][j];
-  out[e * width + c0 + j] = sum;
+    for (int w = 1; w < WAVES; ++w) sum += part[w][j];
+    out[e * width + c0 + j] = sum;
+  }
 }
 
 // d_weights[r] += sum_c dy[src(r)][c] bias[e(r)][c]: one wave a row, lanes 8 columns a
@@ -667,12 +666,28 @@ int expert_sums(const char* name, const T* x, const int32_t* index, int32_t inde
   if (int rc = experts_ok(name, offsets, experts)) return rc;
   BUX_CHECK(out != nullptr && (m == 0 || x != nullptr), "%s: NULL buffer", name);
   // every expert's sum is written (0 for none); rows at or past m add nothing
-  const int64_t chunks = ceil_div(width, SUM_COLS);
-  BUX_CHECK(experts * chunks < (1LL << 31), "%s: too large", name);
-  hipLaunchKernelGGL(expert_sums_kernel<T>, dim3(static_cast<unsigned>(experts * chunks)),
-                     dim3(SUM_THREADS), 0, as_stream(stream), x, index, index_div, sources, weights,
-                     m, width, offsets, experts, out);
-  return launched("expert_sums_kernel");
+  auto go = [&](auto kernel, int waves, int columns) {
+    const int64_t blocks = experts * ceil_div(width, columns);
+    BUX_CHECK(blocks < (1LL << 31), "%s: too large", name);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(waves * 64), 0,
+                       as_stream(stream), x, index, index_div, sources, weights, m, width, offsets,
+                       experts, out);
+    return launched("expert_sums_kernel");
+  };
+  // What bounds a sum is the rows its waves add one after another, while there are too few
+  // workgroups to fill the chip or one expert has most of the rows; past that, wide loads; and
+  // with few rows, the waves to start. us, 4 waves of 512 columns a row at a time / 8 waves, 2
+  // rows / 16 waves of 256 columns, 4 rows / 16 waves of 512 columns, 2 rows:
+  //   bfloat16, 128 experts, 1600 rows of 2880       4.3 /  4.3 /  7.9 /  5.2
+  //   float32, 16 experts, 4004 rows of 1024        15.1 /  8.0 /  5.4 /  6.6
+  //   bfloat16, 8 experts, 65536 rows of 256         521 /  241 /  120 /  144
+  //   bfloat16, 32 experts, 16384 rows of 4096        56 /   32 /   22 /   29
+  //   bfloat16, 128 experts, 32768 rows of 5760       66 /   72 /   87 /   69
+  //   by index, 256 experts, 65536 rows of 7168      265 /  257 /  404 /  260
+  //   on Zipf loads, 128 experts, 32768 of 2880      805 /  445 /  240 /  240
+  if (m <= 32 * static_cast<int64_t>(experts)) return go(expert_sums_kernel<T, 8, 8, 2>, 8, 512);
+  if (experts * ceil_div(width, 256) <= 512) return go(expert_sums_kernel<T, 16, 4, 4>, 16, 256);
+  return go(expert_sums_kernel<T, 16, 8, 2>, 16, 512);
 }
 
 template <typename T>

@@ -85,3 +85,12 @@ def test_norm_gradients_of_every_row(lib, m, d):
     torch.cuda.synchronize()
     for i in range(2):
         assert torch.equal(got[i], torch.cat([p[i] for p in parts]))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("sizes,width", [([7, 0, 8, 15, 33, 1], 520), ([32] * 6, 1288),
+                                         ([31, 32, 33, 100, 0, 17] * 20, 1288), ([40, 41] * 64, 1032)])
+def test_expert_sums_in_each_form(lib, sizes, width, dtype):
+    """Few rows an expert (8 waves of 512 columns), and many in more workgroups than the 512
+    up to which 16 waves take 256 columns: around a turn of the waves and the columns' ends."""
+    test_expert_sums(lib, sizes, width, dtype)
