@@ -12,7 +12,7 @@
 //               by expert, and their gradients
 //
 // All HBM-streaming: a lane moves 16 bytes (8 bfloat16) a load; a workgroup of 256
-// lanes takes 2048 columns of a row. The activation computes in float32 and rounds
+// lanes takes 2048 columns of a row (the sums: sums_threads). The activation computes in float32 and rounds
 // once to bfloat16 (XLA fuses the elementwise chain and keeps float32 inside).
 
 #include <type_traits>
@@ -110,14 +110,26 @@ __global__ __launch_bounds__(THREADS) void token_rows_narrow_kernel(
   rows[e] = token < 0 ? uint16_t{0} : z[token * width + c];
 }
 
-// A token's columns go to as few workgroups as hold them, each of at most SUMS_MOST
-// threads and as even as whole waves allow (2880 columns: 6 waves, not two workgroups of 4
-// of which the second has 1.6 to do; 8192 biased sums of 4 picks 95 -> 85 us).
-constexpr int SUMS_MOST = 512;
+// A token's columns go to workgroups of the most waves, up to 4, that leave none idle, or of
+// 6 that hold them all: idle waves cost a launch each, and uneven workgroups (5 waves) the
+// CUs' balance. us, 4 waves / as few workgroups of up to 8 as hold a row / these: 8192
+// bfloat16 biased sums of 4 picks, 2880 columns 72 / 62 / 62 (6 waves); 8192 float32 sums of a
+// pick, 4104 columns 54 / 62 / 54 (3 waves); 4096 biased sums of 6 picks, 6400 columns 110 /
+// 110 / 103 (a wave); 8192 of 8 picks, 2048 columns 81 / 82 / 81 (4 waves).
+constexpr int SUMS_MOST = 384;
 int sums_threads(int64_t width) {
-  const int64_t vecs = ceil_div(width, VEC), groups = ceil_div(vecs, SUMS_MOST);
-  return static_cast<int>(ceil_div(ceil_div(vecs, groups), 64) * 64);
+  const int64_t waves = ceil_div(width, 64 * VEC);
+  if (waves == 6) return 384;
+  for (int w = 4; w > 1; --w)
+    if (waves % w == 0) return 64 * w;
+  return 64;
 }
+// A token's columns in `chunks` workgroups of `span`: arguments, since a kernel reads its
+// launch's dimensions through one more load, and divides by them (8192 bfloat16 sums of a pick,
+// 2048 columns: 16.9 us with both, 15.3 with neither).
+struct Cut {
+  uint32_t chunks, span;
+};
 
 // KMAX > 0: the token's k <= KMAX picks' rows are all requested before the first is
 // added (their indices first, then their rows); KMAX = 0: any k, one pick at a time.
@@ -158,13 +170,11 @@ template <int KMAX, bool BIAS>
 __global__ __launch_bounds__(SUMS_MOST) void token_sums_kernel(const uint16_t* __restrict__ y,
                                                              int64_t y_rows,
                                                              const int32_t* __restrict__ inverse,
-                                                             int32_t k, int64_t width,
+                                                             int32_t k, int64_t width, Cut cut,
                                                              PickBias<uint16_t> pb,
                                                              uint16_t* __restrict__ out) {
-  const int64_t span = static_cast<int64_t>(blockDim.x) * VEC;  // sums_threads's
-  const int64_t chunks = (width + span - 1) / span;
-  const int64_t t = blockIdx.x / chunks;
-  const int64_t c = (blockIdx.x % chunks) * span + threadIdx.x * VEC;
+  const int64_t t = blockIdx.x / cut.chunks;
+  const int64_t c = static_cast<int64_t>(blockIdx.x % cut.chunks) * cut.span + threadIdx.x * VEC;
   if (c >= width && !(BIAS && KMAX > 0)) return;  // experts_of takes whole waves
   float acc[VEC];
 #pragma unroll
@@ -253,15 +263,13 @@ template <int KMAX, bool BIAS>
 __global__ __launch_bounds__(SUMS_MOST) void token_sums_f32_kernel(const float* __restrict__ y,
                                                                  int64_t y_rows,
                                                                  const int32_t* __restrict__ inverse,
-                                                                 int32_t k, int64_t width,
+                                                                 int32_t k, int64_t width, Cut cut,
                                                                  PickBias<float> pb,
                                                                  float* __restrict__ out) {
   // Each product rounds before it is added, as the reference's ops do (no FMA contraction).
 #pragma clang fp contract(off)
-  const int64_t span = static_cast<int64_t>(blockDim.x) * VEC;  // sums_threads's
-  const int64_t chunks = (width + span - 1) / span;
-  const int64_t t = blockIdx.x / chunks;
-  const int64_t c = (blockIdx.x % chunks) * span + threadIdx.x * VEC;
+  const int64_t t = blockIdx.x / cut.chunks;
+  const int64_t c = static_cast<int64_t>(blockIdx.x % cut.chunks) * cut.span + threadIdx.x * VEC;
   if (c >= width && !(BIAS && KMAX > 0)) return;  // experts_of takes whole waves
   float4 acc[2] = {make_float4(0, 0, 0, 0), make_float4(0, 0, 0, 0)};
   auto add = [&](const float4* row) {
@@ -578,26 +586,27 @@ int token_sums(const char* name, const uint16_t* y, int64_t y_rows, const int32_
   if (tokens == 0) return BUX_OK;
   BUX_CHECK(y && inverse && out, "%s: NULL buffer", name);
   const int threads = sums_threads(width);
-  const int64_t blocks = tokens * ceil_div(width, threads * VEC);
+  const int64_t chunks = ceil_div(width, threads * VEC), blocks = tokens * chunks;
   BUX_CHECK(blocks < (1LL << 31), "%s: too large", name);
   dim3 grid(static_cast<unsigned>(blocks));
+  const Cut cut{static_cast<uint32_t>(chunks), static_cast<uint32_t>(threads * VEC)};
   const PickBias<uint16_t> none{nullptr, nullptr, 0, nullptr};
   hipStream_t s = as_stream(stream);
   if (pb && k <= 4)
     hipLaunchKernelGGL((token_sums_kernel<4, true>), grid, dim3(threads), 0, s, y, y_rows,
-                       inverse, k, width, *pb, out);
+                       inverse, k, width, cut, *pb, out);
   else if (pb && k <= 8)
     hipLaunchKernelGGL((token_sums_kernel<8, true>), grid, dim3(threads), 0, s, y, y_rows,
-                       inverse, k, width, *pb, out);
+                       inverse, k, width, cut, *pb, out);
   else if (pb)
     hipLaunchKernelGGL((token_sums_kernel<0, true>), grid, dim3(threads), 0, s, y, y_rows,
-                       inverse, k, width, *pb, out);
+                       inverse, k, width, cut, *pb, out);
   else if (k <= 8)
     hipLaunchKernelGGL((token_sums_kernel<8, false>), grid, dim3(threads), 0, s, y, y_rows,
-                       inverse, k, width, none, out);
+                       inverse, k, width, cut, none, out);
   else
     hipLaunchKernelGGL((token_sums_kernel<0, false>), grid, dim3(threads), 0, s, y, y_rows,
-                       inverse, k, width, none, out);
+                       inverse, k, width, cut, none, out);
   return launched("token_sums_kernel");
 }
 
@@ -612,23 +621,27 @@ int token_sums_f32(const char* name, const float* y, int64_t y_rows, const int32
   if (tokens == 0) return BUX_OK;
   BUX_CHECK(y && inverse && out, "%s: NULL buffer", name);
   const int threads = sums_threads(width);
-  const int64_t blocks = tokens * ceil_div(width, threads * VEC);
+  const int64_t chunks = ceil_div(width, threads * VEC), blocks = tokens * chunks;
   BUX_CHECK(blocks < (1LL << 31), "%s: too large", name);
   dim3 grid(static_cast<unsigned>(blocks));
+  const Cut cut{static_cast<uint32_t>(chunks), static_cast<uint32_t>(threads * VEC)};
   hipStream_t s = as_stream(stream);
   const PickBias<float> none{nullptr, nullptr, 0, nullptr};
-  if (pb && k <= 8)
+  if (pb && k <= 4)
+    hipLaunchKernelGGL((token_sums_f32_kernel<4, true>), grid, dim3(threads), 0, s, y, y_rows,
+                       inverse, k, width, cut, *pb, out);
+  else if (pb && k <= 8)
     hipLaunchKernelGGL((token_sums_f32_kernel<8, true>), grid, dim3(threads), 0, s, y, y_rows,
-                       inverse, k, width, *pb, out);
+                       inverse, k, width, cut, *pb, out);
   else if (pb)
     hipLaunchKernelGGL((token_sums_f32_kernel<0, true>), grid, dim3(threads), 0, s, y, y_rows,
-                       inverse, k, width, *pb, out);
+                       inverse, k, width, cut, *pb, out);
   else if (k <= 8)
     hipLaunchKernelGGL((token_sums_f32_kernel<8, false>), grid, dim3(threads), 0, s, y, y_rows,
-                       inverse, k, width, none, out);
+                       inverse, k, width, cut, none, out);
   else
     hipLaunchKernelGGL((token_sums_f32_kernel<0, false>), grid, dim3(threads), 0, s, y, y_rows,
-                       inverse, k, width, none, out);
+                       inverse, k, width, cut, none, out);
   return launched("token_sums_f32_kernel");
 }
 

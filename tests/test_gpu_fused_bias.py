@@ -69,3 +69,26 @@ def test_biased_token_sums(lib, k, experts, width, dtype):
     size = (y[rows].double() * there).abs().sum(1) + part.abs().sum(1)
     bound = k * 2.0**-24 * size + unit * (both[0].abs() + both[1].abs()) + unit * sum(both).abs()
     assert bool(((got.double() - sum(both)).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", [8, 504, 520, 1024, 1536, 2560, 2880, 3072, 4104, 6400])
+def test_token_sums_of_any_width(lib, width, dtype):
+    """The workgroups' waves, 1 to 4 or 6, and the columns' end in them: the sums with and
+    without biases of rows whose values their sums hold exactly."""
+    from bux_amd import moe
+    g = torch.Generator(device="cuda").manual_seed(102)
+    t, k, e = 19, 3, 7
+    idx = torch.randint(0, e, (t, k), generator=g, device="cuda").int()
+    s = moe.sort_by_expert(idx, e)
+    y, bias = (torch.randint(-8, 9, shape, generator=g, device="cuda").to(dtype)
+               for shape in ((t * k, width), (e, width)))
+    w = torch.randint(1, 3, (t * k,), generator=g, device="cuda").to(dtype)
+    inverse = s.inverse.view(t, k)
+    announce("token sums", width, dtype)
+    plain = moe.sum_by_token(y, inverse)
+    biased = moe.sum_by_token_biased(y, inverse, bias, s.offsets, w)
+    torch.cuda.synchronize()
+    want = y[inverse.long()].sum(1)
+    assert torch.equal(plain, want)
+    assert torch.equal(biased, want + (bias[idx.long()] * w[inverse.long()][..., None]).sum(1))
