@@ -187,16 +187,30 @@ int launch_as(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b
 
 }  // namespace
 
-// The line between the two kernels, by the mean rows a group (the sizes are the device's)
-// and whether the tiled one's 256-column tiles fill half of the chip. Measured against
-// grouped_mx.hip's (us; even loads, then Zipf(1.2)): 128 groups of K 2048, N 1536, half a row
-// a group 53 -> 29, 28 -> 21; 6 rows 90 -> 73, 83 -> 67; 16 rows 88 -> 77, 87 -> 89; 26 rows 90
-// -> 93, 107 -> 106; 16 groups of K 6400, N 4096, 6 rows 90 -> 76, 89 -> 85; 16 rows 88 -> 78, 86
-// -> 96; 32 rows 86 -> 106. Few tiles: 8 groups of K 7168, N 4096, 12 rows 80 -> 44, 32 rows 80
-// -> 55; of K 2048, N 1536, 32 rows 27 -> 13.
+// The line between the two kernels, by what the host knows, rows, groups and columns; how the
+// rows fall on the groups is the device's. A group of more than a block of rows has its B read
+// once a block here and once a tile of 256 rows by grouped_mx.hip, so rows crowded into few
+// groups are what the line must bear: below it no load measured slower (even, Zipf(1.2), half
+// of the rows with one group, all with one, with a fifth of the groups, groups of 33 and of
+// 65 rows). Either the tiles of even full groups would fill at most half of the chip, up to a
+// block of rows a group; or the tiles that the rows could fill in blocks of 32, crowded or
+// not, are a quarter of its CUs. us, grouped_mx.hip's and this (even; all rows with one group;
+// groups of 33 rows, each a second block of one row):
+//   128 groups of K 2048, N 1536, 320 rows (60 tiles)     103 and  74;  27 and 15;  28 and 13
+//   128 of K 768, N 2048, 256 rows (64)                    56 and  43;  14 and 12;  14 and 12
+//   16 of K 6400, N 4096, 128 rows (64; Zipf 88 and 86)   100 and  82;  71 and 26;  71 and 27
+//   256 of K 7168, N 4096, 128 rows (64)                  736 and 626;  78 and 40;  78 and 62
+//   8 of K 7168, N 4096, 256 rows (few tiles)              83 and  44;  63 and 46;  83 and 62
+// and past it even loads gain as before, crowded ones lose:
+//   128 of K 2048, N 1536, 1024 rows (192)                100 and  77;  24 and 21;  29 and 35
+//   16 of K 6400, N 4096, 256 rows (128; Zipf 91 and 100)  99 and  81;  58 and 43;  74 and 56
+//   128 of K 2944, N 5760, 256 rows (184)                 464 and 386;  31 and 40;  37 and 51
+//   256 of K 2048, N 7168, 192 rows (168)                 585 and 494;  25 and 41;  28 and 56
 bool rows_direct(int64_t m, int32_t groups, int64_t n) {
-  const bool few = groups * ceil_div(n, BN) <= 128;
-  return m > 0 && m <= (few ? 32 : 16) * static_cast<int64_t>(groups);
+  const int64_t tiles = ceil_div(n, BN);
+  if (m <= 0) return false;
+  if (groups * tiles <= 128) return m <= DIRECT_BLOCK * static_cast<int64_t>(groups);
+  return m <= 16 * static_cast<int64_t>(groups) && ceil_div(m, DIRECT_BLOCK) * tiles <= 64;
 }
 
 int launch_rows_direct(const uint8_t* a_values, const uint8_t* a_scales, const uint8_t* b_values,
@@ -211,3 +225,8 @@ int launch_rows_direct(const uint8_t* a_values, const uint8_t* a_scales, const u
 }
 
 }  // namespace bux
+
+// Which kernel a call takes, for tests alone (not in bux_amd.h: the line may move).
+extern "C" int bux_rows_direct(int64_t m, int32_t groups, int64_t n) {
+  return bux::rows_direct(m, groups, n);
+}

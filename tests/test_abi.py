@@ -427,3 +427,22 @@ def test_biased_rows_reject_bad_arguments(lib):
     assert rows(k=100) == 1 and "k=100" in _msg(lib)
     assert rows(values=None) == 1 and "NULL buffer" in _msg(lib)
     assert "bux_mx_grouped_rows_biased" in _msg(lib)
+
+
+def _direct(lib, m: int, groups: int, n: int) -> bool:
+    """Whether a rows GEMM goes to rows_direct_kernel (the library's own rule)."""
+    return bool(lib.bux_rows_direct(ctypes.c_int64(m), groups, ctypes.c_int64(n)))
+
+
+# groups, n, the most rows that go to the kernel for few rows
+@pytest.mark.parametrize("groups,n,most", [
+    (8, 4096, 256), (128, 256, 4096), (1, 32768, 32),  # 128 tiles of full groups: a block a group
+    (129, 256, 2048), (9, 4096, 128), (128, 1536, 320), (128, 2048, 256), (256, 7168, 64),
+    (5, 6656, 64), (3, 12288, 32), (256, 16384, 32),  # 64 tiles of 32 rows
+    (3, 16640, 0), (256, 16640, 0)])
+def test_the_line_of_the_kernel_for_few_rows(lib, groups, n, most):
+    """Where rows crowded into few groups would make the kernel for few rows the slower one,
+    no call goes to it."""
+    assert not _direct(lib, 0, groups, n)
+    assert all(_direct(lib, m, groups, n) == (m <= most)
+               for m in {1, 2, most // 2 or 1, most or 1, most + 1, most + 31, 2 * most + 1, 100000})

@@ -92,3 +92,8 @@ def test_token_sums_of_any_width(lib, width, dtype):
     want = y[inverse.long()].sum(1)
     assert torch.equal(plain, want)
     assert torch.equal(biased, want + (bias[idx.long()] * w[inverse.long()][..., None]).sum(1))
+
+
+def test_the_biased_case_of_few_rows_takes_its_kernel(lib):
+    from tests.test_abi import _direct
+    assert _direct(lib, 103 + 30, 63, 132) and not _direct(lib, 685 + 30, 4, 512)

@@ -75,3 +75,13 @@ def test_float32_outputs_round_to_the_bfloat16_ones(lib, sizes, k, n):
     for b16, f32 in (rows, dw):
         assert torch.equal(b16, f32.to(torch.bfloat16))
     assert bool((dw[1] != 0).any(-1).all()) and bool((rows[1][:sum(sizes)] != 0).any(-1).all())
+
+
+@pytest.mark.parametrize("sizes,k,n", [c for c in SMALL if len(c[0]) < 128] + [([3] * 64, 640, 1540)])
+def test_the_two_rows_kernels_each_take_their_call(lib, sizes, k, n):
+    """The comparison above, with the library's own rule saying that the call of few rows
+    takes rows_direct_kernel and the other the tiled one."""
+    from tests.test_abi import _direct
+    groups, m = len(sizes), sum(sizes) + 3
+    assert _direct(lib, m, groups, n) and not _direct(lib, 32 * groups + 1, groups, n)
+    test_rows_of_few_rows_are_the_tiled_kernels(lib, sizes, k, n)
