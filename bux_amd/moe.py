@@ -69,6 +69,8 @@ def sort_for_layer(
     """Return `sort_by_expert`, `picked_weights` of it and, with `height`, the MXFP8 GEMMs'
     `tiles_of` its sizes (a of `height` rows, outputs of the picks), in the sort's own
     kernels. weights: bfloat16 or float32, one a pick."""
+    if weights.dtype not in (torch.bfloat16, torch.float32):
+        raise TypeError(f"sort_for_layer: bfloat16 or float32 weights, not {weights.dtype}")
     n = idx.numel()
     weights = weights.reshape(-1)
     if weights.numel() != n:  # picks past the weights weigh 0

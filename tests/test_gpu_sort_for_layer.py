@@ -78,3 +78,12 @@ def test_picks_of_few_experts(lib, n):
         np.testing.assert_array_equal(s.inverse.cpu().numpy(), want.inverse)
         np.testing.assert_array_equal(s.sizes.cpu().numpy(), want.sizes)
         assert torch.equal(row_weights, weights.reshape(-1)[s.order.long()])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.int32, torch.float64])
+def test_weights_of_other_dtypes_are_refused(lib, dtype):
+    from bux_amd import moe
+    idx = to_gpu(np.array([[1, 0]], np.int32))
+    announce("layer sort, weights of another dtype", dtype)
+    with pytest.raises(TypeError, match="weights"):
+        moe.sort_for_layer(idx, 2, torch.ones(1, 2, dtype=dtype, device="cuda"), None)
