@@ -643,7 +643,7 @@ def experts_forward(
             if fprop:  # the bias in the GEMM's epilogue
                 projected = grouped_mxfp8.rows(
                     x_k, up_k, s.sizes, dt, height=m, tiles=listed,
-                    bias=None if up_bias is None else up_bias.reshape(e, f * p).contiguous())
+                    bias=None if up_bias is None else up_bias.reshape(e, f * p))
             else:
                 projected = grouped.dot(rows, up2, s.sizes, tiles=plain)
         if up_bias is not None and not fprop:

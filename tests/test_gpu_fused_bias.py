@@ -97,3 +97,22 @@ def test_token_sums_of_any_width(lib, width, dtype):
 def test_the_biased_case_of_few_rows_takes_its_kernel(lib):
     from tests.test_abi import _direct
     assert _direct(lib, 103 + 30, 63, 132) and not _direct(lib, 685 + 30, 4, 512)
+
+
+@pytest.mark.parametrize("fmt", ["mxfp8", "compute"])
+def test_a_strided_up_bias_is_refused(lib, fmt):
+    """Every other expert's biases of a larger tensor: refused where the bias rides the GEMM
+    as where it is an op of its own."""
+    from bux_amd import moe
+    t, k, e, d, f = 16, 2, 4, 128, 64
+    g = torch.Generator(device="cuda").manual_seed(103)
+    z, up, down = ((torch.randn(*s, generator=g, device="cuda") * 0.1).bfloat16()
+                   for s in ((t, d), (e, d, f, 2), (e, f, d)))
+    idx = torch.randint(0, e, (t, k), generator=g, device="cuda").int()
+    w = torch.full((t, k), 0.5, device="cuda").bfloat16()
+    biases = torch.randn(2 * e, f, 2, generator=g, device="cuda").bfloat16()
+    announce("a strided up bias", fmt)
+    moe.experts_forward(z, idx, w, up, down, fmt=fmt, up_bias=biases[::2].contiguous())
+    with pytest.raises(ValueError, match="contiguous"):
+        moe.experts_forward(z, idx, w, up, down, fmt=fmt, up_bias=biases[::2])
+    torch.cuda.synchronize()
