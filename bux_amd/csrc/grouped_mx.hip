@@ -451,7 +451,6 @@ __device__ void store_f32(const Values& values, float* tile, int32_t ld, int32_t
 constexpr int PITCH = 272;
 static_assert(4 * 32 * PITCH == sizeof(Stage), "the epilogue's regions fill a stage");
 
-// With LO, only the rows from row_lo on are stored.
 // The accumulators of a 32 x 32 block as bfloat16 pairs: run g's columns 0-1 and 2-3
 // (v_cvt_pk_bf16_f32: two floats to two bfloat16, nearest even).
 __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {

@@ -36,8 +36,9 @@
 //     different banks.
 // bfloat16 blocks are reduced and converted as packed pairs (common.h's e4m3x4_bf16): the
 // quantizers by index and of the activations' gradients issued too many VALU instructions to
-// keep up with memory (config 3: the tokens by index 171 -> 153 us, h 126 -> 121, d projected
-// 233 -> 215, W_up 283 -> 280; DeepSeek-V3's tokens 300 -> 291).
+// keep up with memory (by themselves, config 3: the tokens by index 156 -> 141 us, h 122 ->
+// 120, d projected 217 -> 215; DeepSeek-V3's tokens 247 -> 220; the weights, at HBM's rate,
+// 283 both).
 // HBM traffic per element: 2 bytes read (4 of float32), 2 x (1 + 1/32) bytes written; the
 // codes go out as non-temporal stores (below).
 //
