@@ -13,9 +13,9 @@ __host__ __device__ __forceinline__ int64_t direct_row(int32_t lo, uint32_t i) {
   return lo + static_cast<int64_t>(DIRECT_BLOCK) * i;
 }
 
-// Whether a rows GEMM of `m` rows in `groups` groups, `n` columns, goes to
-// rows_direct_kernel.
-bool rows_direct(int64_t m, int32_t groups, int64_t n);
+// The blocks of rows a wave of rows_direct_kernel takes of a rows GEMM of `m` rows in
+// `groups` groups, `n` columns: 1 or 2, or 0 where the call is grouped_mx.hip's.
+int rows_direct(int64_t m, int32_t groups, int64_t n);
 
 // As grouped_mx.hip's launch_rows: `list` a tile list of `slots` records (its starts
 // before them), the operands in the tiled layout, `bias` NULL or

@@ -429,20 +429,23 @@ def test_biased_rows_reject_bad_arguments(lib):
     assert "bux_mx_grouped_rows_biased" in _msg(lib)
 
 
-def _direct(lib, m: int, groups: int, n: int) -> bool:
-    """Whether a rows GEMM goes to rows_direct_kernel (the library's own rule)."""
-    return bool(lib.bux_rows_direct(ctypes.c_int64(m), groups, ctypes.c_int64(n)))
+def _direct(lib, m: int, groups: int, n: int) -> int:
+    """The blocks of 32 rows that a wave of rows_direct_kernel takes of a rows GEMM (the
+    library's own rule), 0 where the call goes to the tiled kernel."""
+    return lib.bux_rows_direct(ctypes.c_int64(m), groups, ctypes.c_int64(n))
 
 
-# groups, n, the most rows that go to the kernel for few rows
-@pytest.mark.parametrize("groups,n,most", [
-    (8, 4096, 256), (128, 256, 4096), (1, 32768, 32),  # 128 tiles of full groups: a block a group
-    (129, 256, 2048), (9, 4096, 128), (128, 1536, 320), (128, 2048, 256), (256, 7168, 64),
-    (5, 6656, 64), (3, 12288, 32), (256, 16384, 32),  # 64 tiles of 32 rows
-    (3, 16640, 0), (256, 16640, 0)])
-def test_the_line_of_the_kernel_for_few_rows(lib, groups, n, most):
+# groups, n, the most rows that go to the kernel for few rows, and to its waves of two blocks
+@pytest.mark.parametrize("groups,n,one,two", [
+    (8, 4096, 256, 0), (128, 256, 4096, 0), (1, 32768, 32, 0),  # 128 tiles of full groups: a block a group
+    (129, 256, 2048, 2064), (9, 4096, 128, 144), (5, 6656, 64, 80), (3, 12288, 32, 48),
+    (3, 16640, 0, 48),  # 64 tiles of 32 rows, then 16 rows a group
+    (128, 1536, 320, 2048), (128, 2048, 256, 2048), (64, 2304, 224, 1024),
+    (256, 7168, 64, 576), (256, 16384, 32, 256), (256, 16640, 0, 224)])  # then 512 tiles
+def test_the_line_of_the_kernel_for_few_rows(lib, groups, n, one, two):
     """Where rows crowded into few groups would make the kernel for few rows the slower one,
-    no call goes to it."""
-    assert not _direct(lib, 0, groups, n)
-    assert all(_direct(lib, m, groups, n) == (m <= most)
-               for m in {1, 2, most // 2 or 1, most or 1, most + 1, most + 31, 2 * most + 1, 100000})
+    no call goes to it, or to waves of two blocks, and none far past it."""
+    edges = {x for y in (one, two) for x in (y // 2, y, y + 1, y + 31)} | {1, 2, 2 * one + 1, 100000}
+    for m in edges:
+        want = 0 if m < 1 else 1 if m <= one else 2 if m <= two else 0
+        assert _direct(lib, m, groups, n) == want, m

@@ -83,5 +83,33 @@ def test_the_two_rows_kernels_each_take_their_call(lib, sizes, k, n):
     takes rows_direct_kernel and the other the tiled one."""
     from tests.test_abi import _direct
     groups, m = len(sizes), sum(sizes) + 3
-    assert _direct(lib, m, groups, n) and not _direct(lib, 32 * groups + 1, groups, n)
+    assert _direct(lib, m, groups, n) == 1 and _direct(lib, 32 * groups + 1, groups, n) == 0
     test_rows_of_few_rows_are_the_tiled_kernels(lib, sizes, k, n)
+
+
+# groups of a block of rows, of two, of more, in part and whole; a tile and a second one
+CROWDED = [33, 64, 65, 0, 1, 300, 31, 32, 128, 97] + [2] * 54
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("k,n", [(128, 2308), (256, 2304), (384, 2500), (640, 2308)])
+def test_waves_of_two_blocks_are_the_tiled_kernel(lib, k, n, dtype):
+    """K of one pair to five, columns off the waves' 64, with and without a bias."""
+    from bux_amd import grouped_mxfp8
+    from tests.test_abi import _direct
+    rng = np.random.default_rng(72)
+    groups, filled = len(CROWDED), sum(CROWDED)
+    m, far = filled + 3, 32 * groups + 1
+    assert _direct(lib, m, groups, n) == 2 and _direct(lib, far, groups, n) == 0
+    a = _codes(rng, (far, k))
+    few = grouped_mxfp8.Tiled(a.values[:, :m].contiguous(), a.scales[:, :m].contiguous())
+    b = _codes(rng, (groups, n, k))
+    gs = torch.tensor(CROWDED, dtype=torch.int32, device="cuda")
+    bias = (torch.randn(groups, n, device="cuda") * 100).to(dtype)
+    announce("waves of two blocks", k, n, dtype)
+    for added in (None, bias):
+        got, want = (grouped_mxfp8.rows(x, b, gs, dtype, tiles=grouped_mxfp8.tiles_of(gs, rows, rows),
+                                        bias=added) for x, rows in ((few, m), (a, far)))
+        torch.cuda.synchronize()
+        assert torch.equal(got, want[:m])
+        assert (got[filled:] == 0).all() and bool((got[:filled] != 0).any(-1).all())
